@@ -5,6 +5,7 @@
 #include <stdarg.h>
 
 #include "dfm_common.h"
+#include "radon_bp.h"
 
 namespace dfm {
 
@@ -966,17 +967,22 @@ int dfm_radon_backward_table(const float* sino, float* img_k, const int32_t* pta
                 "dfm_radon_backward_table: bad sizes");
   // variant = 4: a workgroup per 4x4 tile and channel block (4 angles per pass; modes 0 and 1), or ACH + 64 G with
   // ACH 4 or 8 and G 2, 4 or 8: a workgroup per 4x4 tile and G channel blocks, the tile's tables staged once;
-  // + 1024: 8x8 tiles (tbase then holds the 8x8 tiles' first bins), ACH 4 or 8, G 1, 2 or 4
+  // + 1024: 8x8 tiles (tbase then holds the 8x8 tiles' first bins), ACH 4 or 8, G 1, 2 or 4; 4 + 64 + 2048: 8x8 tiles on
+  // the matrix cores (at most 12 bins a tile, 4 a 2x2 quad of pixels)
   const int ach = variant % 64, grp = (variant / 64) % 16, t8 = (variant / 1024) % 4;
   DFM_CHECK_ARG(variant < 4096 &&
                     ((t8 == 0 && grp == 0 && ach == 4) ||
                      (t8 == 0 && (grp == 2 || grp == 4 || grp == 8) && (ach == 4 || ach == 8)) ||
-                     (t8 == 1 && (grp == 1 || grp == 2 || grp == 4) && (ach == 4 || ach == 8))),
+                     (t8 == 1 && (grp == 1 || grp == 2 || grp == 4) && (ach == 4 || ach == 8)) ||
+                     (t8 == 2 && grp == 1 && ach == 4)),
                 "dfm_radon_backward_table: variant %d: 4, or 4 / 8 + 64 G for G = 2, 4, 8 channel blocks per "
-                "workgroup, or 4 / 8 + 64 G + 1024 (8x8 tiles, G = 1, 2, 4)",
+                "workgroup, or 4 / 8 + 64 G + 1024 (8x8 tiles, G = 1, 2, 4), or 4 + 64 + 2048 (matrix cores)",
                 variant);
   if (k_n == 0) return DFM_OK;
   const int k4n = k_n / 4;
+  if (t8 == 2)
+    return dfm::launch_backward_mfma(sino, img_k, bgeo, tbase, nx, ny, ns, n_angles, kstride / 4, k_off / 4, k4n,
+                                     skstride / 4, x, z, T, inv_p, lam, mode, (hipStream_t)stream);
   const int ntiles = ((nx + 3) / 4) * ((ny + 3) / 4);
   if (t8) {
     const int ntiles8 = ((nx + 7) / 8) * ((ny + 7) / 8);

@@ -24,6 +24,7 @@ from .crystallography import Material, group_reflections_into_rings
 from .quadrature import DEFAULT_TOL, QuadratureRule, setup_quadrature  # noqa: F401
 from .support import fov_support_mask
 
+BWD_MFMA = 4 + 64 + 2048    # the matrix-core variant of dfm_radon_backward_table
 KEV_ANGSTROM = 12.398       # single_phase_forward_operator.py:554
 AUTO_FFT_PIXELS = 400 * 400
 
@@ -164,6 +165,9 @@ def radon_tables(geo64, idx, nx, ny, ns, radon_scale, n_bands=1):
         np.minimum.at(base8[a], tile8, lo[a])
         np.maximum.at(top8[a], tile8, hi[a])
     tbase8 = base8.astype(np.int32) if not np.any(top8 - base8 >= 16) else np.full((1, 1), -1, np.int32)
+    # the matrix-core backprojection: at most 12 bins an 8 x 8 tile and 4 a 2 x 2 quad of pixels
+    mfma_ok = bool(not np.any(top8 - base8 >= 12) and
+                   np.all(np.abs(g["X"][idx]) + np.abs(g["Y"][idx]) < 2.0 - 1e-9))
     # line sweep: per angle the sweep class (0: image rows, |X| >= |Y|; 1: image columns) and its float64 geometry
     cls = (np.abs(g["X"][idx]) < np.abs(g["Y"][idx])).astype(np.int32)
     bh = -(-ny // n_bands)
@@ -189,7 +193,7 @@ def radon_tables(geo64, idx, nx, ny, ns, radon_scale, n_bands=1):
     sweep_grp_p, sweep_gcls_p = sweep_groups(512, -(-ns // 2)) if pairs_ok else (np.full((1, 1), -1, np.int32),
                                                                          np.zeros(1, np.int32))
     return {"row_ptr": row_ptr.astype(np.int32), "pix": pix[order].astype(np.int32), "band_ptr": band_ptr.astype(np.int32),
-            "tbase8": tbase8,
+            "tbase8": tbase8, "mfma_ok": mfma_ok,
             "sweep_geo": np.stack([g["X"][idx], g["Y"][idx], g["T0"][idx], g["hw"][idx], g["top"][idx],
                                    radon_scale * g["inv_a"][idx]], 1).astype(np.float64),
             # the backprojection's per-angle geometry (X, Y, T0, hw, top, w / A): the grouped kernels derive the
@@ -433,8 +437,8 @@ class SinglePhaseForwardOperator:
         self._geo_angles = {id(self.geo_fwd): (self.geo_fwd, all_a), id(self.geo_bwd): (self.geo_bwd, all_a)}
         # kernel choices (identical results up to float32 rounding; set by autotune): forward "table" (geometry
         # tables, 2 taps), "band", "sweep", "psweep" (line sweeps), "arith" (footprint arithmetic, any taps);
-        # backward "table" (tile and grouped forms by variant number) or "arith"
-        self.radon_variant = {"fwd": 8 + 256, "bwd": 4 + 64 * 4, "fwd_kernel": "table", "bwd_kernel": "table"}
+        # backward "table" (tile, grouped and matrix-core forms by variant number; None: by size) or "arith"
+        self.radon_variant = {"fwd": 8 + 256, "bwd": None, "fwd_kernel": "table", "bwd_kernel": "table"}
         self.tuning = None
         self.marks = None                       # a list while a profiling pass records per-launch events (mark())
         # image bands of the banded forward projection: one XCD's band of 64 channels within about 2 MB of L2
@@ -1033,9 +1037,25 @@ class SinglePhaseForwardOperator:
         and 3 of dfm_radon_backward_table)."""
         if self.fourier is not None:
             return False
-        v = int(self.radon_variant["bwd"]) if self.radon_variant["bwd"] is not None else 0
-        grouped = (v // 64) % 16 > 0 or (v // 1024) % 4 == 1
-        return self.radon_variant["bwd_kernel"] == "table" and grouped and self._tables(subset) is not None
+        tab = self._tables(subset)
+        if self.radon_variant["bwd_kernel"] != "table" or tab is None:
+            return False
+        v = self._bwd_variant(tab, CH_ALIGN)
+        return (v // 64) % 16 > 0 or (v // 1024) % 4 == 1
+
+    def _bwd_variant(self, tab, kn):
+        """The table backprojection's variant for kn orientation columns: radon_variant["bwd"] if set (by hand or by
+        autotune), else by size. From 32 tiles of 8 x 8 pixels on the matrix-core form (us, SPDHG update, against the
+        best of the others: 99 x 99 x 29760 x 18 angles 1190 / 1344, 99 x 99 x 9920 x 180 2180 / 3130, 99 x 99 x 576 x
+        18 41 / 60, 64 x 64 x 512 x 60 39 / 40). Below that a launch is a chain of passes over the angles and few
+        workgroups: the 8 x 8 form of 8 angles per pass (32 x 32 x 512 x 24: 17 against 20), or for one block of
+        orientations the 4 x 4 form, which has four times the workgroups (16 x 16 x 64 x 30: 16 against 18 and 21)."""
+        v = self.radon_variant["bwd"]
+        if v is not None:
+            return int(v)
+        if -(-self.Nx // 8) * -(-self.Ny // 8) >= 32:
+            return BWD_MFMA if tab["mfma_ok"] else 4 + 64 * 4
+        return 8 + 64 + 1024 if kn > CH_ALIGN and tab["tbase8"].numel() > 1 else 4 + 64 * 4
 
     def _radon_backward(self, sino, geo, tab, n_ang, out_k, kstride, koff, kn, x=None, z=None, T=None, inv_p=0.0,
                         lam=0.0, em=False, pdhg=False):
@@ -1063,13 +1083,16 @@ class SinglePhaseForwardOperator:
         if mode >= 2 and (tab is None or self.radon_variant["bwd_kernel"] != "table"):
             raise ValueError("the fused EM / PDHG updates need a grouped table backprojection (em_fused())")
         if tab is not None and self.radon_variant["bwd_kernel"] != "arith":
-            t8 = (self.radon_variant["bwd"] // 1024) % 4 == 1       # 8x8 tiles: their first-bin table
-            if t8 and tab["tbase8"].numel() == 1:
+            variant = self._bwd_variant(tab, kn)
+            t8 = (variant // 1024) % 4                              # 8x8 tiles: their first-bin table
+            if t8 == 1 and tab["tbase8"].numel() == 1:
                 raise ValueError("8x8 backprojection tiles reach more than 16 bins for this geometry")
+            if t8 == 2 and not tab["mfma_ok"]:
+                raise ValueError("8x8 backprojection tiles reach more than 12 bins for this geometry")
             _lib.call("dfm_radon_backward_table", _lib.ptr(sino), _lib.ptr(out_k), _lib.ptr(tab["ptab"]),
                       _lib.ptr(tab["bp_geo"]), _lib.ptr(tab["tbase8" if t8 else "tbase"]), self.Nx, self.Ny, self.My, n_ang, kstride, koff,
                       kn, kn, _lib.ptr(x),
-                      _lib.ptr(z), _lib.ptr(T), float(inv_p), float(lam), mode, self.radon_variant["bwd"], st)
+                      _lib.ptr(z), _lib.ptr(T), float(inv_p), float(lam), mode, variant, st)
         elif mode == 0:
             _lib.call("dfm_radon_backward", _lib.ptr(sino), _lib.ptr(out_k), _lib.ptr(geo), self.Nx, self.Ny,
                       self.My, n_ang, kstride, koff, kn, kn, self.n_taps, st)
@@ -1138,9 +1161,11 @@ class SinglePhaseForwardOperator:
             elif kern == "psweep":
                 saved["fwd_psweep"] = v
             out["radon_forward"] = (best, times)
-            # the 8x8-tile forms first (the fastest at every measured configuration; the first listed within the
-            # tolerance wins), then the 4x4-tile forms
+            # the matrix-core form first (the fastest at every measured configuration but the smallest; the first listed
+            # within the tolerance wins), then the 8x8-tile and the 4x4-tile forms
             cands = {}
+            if tab["mfma_ok"]:
+                cands["mfma"] = ("table", BWD_MFMA)
             if tab["tbase8"].numel() > 1:
                 cands.update({f"table8:{a}x{g}": ("table", a + 64 * g + 1024)
                               for a, g in ((8, 2), (8, 4), (8, 1), (4, 2), (4, 4), (4, 1))})

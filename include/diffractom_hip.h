@@ -74,7 +74,7 @@ int dfm_radon_backward(const float* sino, float* img_k, const float* geo, int32_
  *   (s0 = floor(t - hw) + 1, s1 = s0 + 1, w = wscale_a / A clamp(hw - |t - s|, 0, top));
  * tile bases tbase (n_angles, ceil(nx/4) * ceil(ny/4)): the first of the 8 bins every 4 x 4 pixel tile reaches.
  * mode 0: img_k = backward(sino); mode 1: the SPDHG primal update of x, z with step T, as dfm_radon_backward_spdhg;
- * mode 2 (grouped variants: + 64 G, + 1024, + 4096 w): the EM update x = T > 0 ? x backward(sino) / (T + lam) : x with
+ * mode 2 (grouped variants: + 64 G, + 1024, + 2048): the EM update x = T > 0 ? x backward(sino) / (T + lam) : x with
  * T the EM sensitivity, lam >= 0, z unused (osem_poisson.py:69-73 osem_update applied to the output of
  * radon_backward_k); mode 3 (grouped variants): the PDHG primal step and extrapolation x' = T > 0 ? max(0, x - T
  * (backward(sino) + lam)) : 0, z = 2 x' - x (x_bar), x = x' (pdhg_poisson.py:69-80 primal_update applied to the
@@ -83,7 +83,9 @@ int dfm_radon_backward(const float* sino, float* img_k, const float* geo, int32_
  * workgroup's table entries staged in LDS), plus 512 q for channel blocks of 64 (q 0) or 128 (q 3) channels;
  * backward: 4, a workgroup per 4 x 4 tile and 64 channels (4 angles staged per pass); or ACH + 64 G (ACH 4 or 8
  * angles per pass; G 2, 4 or 8): a workgroup per tile and G channel blocks, the tile's table rows staged once; + 1024
- * (ACH 4 or 8, G 1, 2 or 4): 8 x 8 tiles, tbase then holding each 8 x 8 tile's first of 16 bins), picked by timing
+ * (ACH 4 or 8, G 1, 2 or 4): 8 x 8 tiles, tbase then holding each 8 x 8 tile's first of 16 bins; 4 + 64 + 2048: 8 x 8
+ * tiles on the FP32 matrix cores, for geometries whose 8 x 8 tiles reach at most 12 bins and whose 2 x 2 quads of
+ * pixels reach at most 4 (|X| + |Y| < 2), tbase as for + 1024), picked by size or by timing
  * (the reference times its tiled / plain projectors the same way, parallel_radon.py:240-281). */
 int dfm_radon_forward_table(const float* img_k, float* sino, const int32_t* row_ptr, const int32_t* ent_pix,
                             const float* ent_w, int32_t ns, int32_t n_angles, int32_t kstride, int32_t k_off,
