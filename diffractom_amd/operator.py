@@ -436,15 +436,15 @@ class SinglePhaseForwardOperator:
         all_a = torch.arange(self.N_Omega, dtype=torch.int32, device=self.device)
         self._geo_angles = {id(self.geo_fwd): (self.geo_fwd, all_a), id(self.geo_bwd): (self.geo_bwd, all_a)}
         # kernel choices (identical results up to float32 rounding; set by autotune): forward "table" (geometry
-        # tables, 2 taps), "band", "sweep", "psweep" (line sweeps), "arith" (footprint arithmetic, any taps);
+        # tables, 2 taps), "band", "sweep", "psweep", "lines" (line sweeps), "arith" (footprint arithmetic, any taps)
+        # or None (by size);
         # backward "table" (tile, grouped and matrix-core forms by variant number; None: by size) or "arith"
-        self.radon_variant = {"fwd": 8 + 256, "bwd": None, "fwd_kernel": "table", "bwd_kernel": "table"}
+        self.radon_variant = {"fwd": 8 + 256, "bwd": None, "fwd_kernel": None, "bwd_kernel": "table"}
         self.tuning = None
         self.marks = None                       # a list while a profiling pass records per-launch events (mark())
         # image bands of the banded forward projection: one XCD's band of 64 channels within about 2 MB of L2
         self.radon_bands = int(min(8, max(1, -(-self.Nx * self.Ny // 8192))))
-        if self.radon_bands >= 4:
-            self.radon_variant["fwd_kernel"] = "band"
+        self._lines_caps = {}
         self._tables_full = self._radon_tables(np.arange(self.N_Omega)) if self.n_taps == 2 else None
 
     def _radon_tables(self, idx):
@@ -1043,6 +1043,47 @@ class SinglePhaseForwardOperator:
         v = self._bwd_variant(tab, CH_ALIGN)
         return (v // 64) % 16 > 0 or (v // 1024) % 4 == 1
 
+    def _fwd_kernel(self, tab, n_angles, kn):
+        """The forward projection's kernel by size, for geometries whose ray pairs the line sweep covers and images of
+        at most 256 x 256 pixels: the line sweep from images of more than 80 pixels a side or 1.5e8 (pixel, orientation,
+        angle) triples on (us, against the table, launches back to back: 99 x 99 x 64 x 18 angles 22 / 37, 88 x 88 x
+        2048 x 6 36 / 56, 64 x 64 x 2048 x 60 68 / 144, 99 x 99 x 9920 x 180 2020 / 4830). Below that its second launch
+        and its chain of lines cost what they save or more (72 x 72 x 512 x 18 31 / 26, 64 x 64 x 6016 x 6 68 / 58, 32 x
+        32 x 512 x 18 17 / 9). Otherwise the table, in bands for large images."""
+        n = max(self.Nx, self.Ny)
+        if tab is not None and tab["pairs_ok"] and n <= 256 and \
+                (n > 80 or self.Nx * self.Ny * n_angles * kn >= 150_000_000):
+            return "lines"
+        return "band" if self.radon_bands >= 4 else "table"
+
+    def _lines_variant(self, tab, kn):
+        """(line ranges, duplicated layout) of the line sweep: radon_variant["fwd_lines"] (ranges + 128 for the
+        duplicated layout) if set by hand or by autotune, else by size. The duplicated layout while two workgroups of
+        it fit a CU's LDS (128 pixels: 99 x 99 x 29760 x 18 angles 0.82 against 0.89 ms; 256 pixels, one workgroup: 1.62
+        against 1.20). With fewer workgroups than CUs the lines are split for two workgroups per CU, in ranges of 8
+        lines or more and at most 12 (99 x 99 x 18 angles: 576 orientations 109 -> 46 us, 2048 117 -> 92 us; 5056, 316
+        workgroups, 178 -> 198)."""
+        v = self.radon_variant.get("fwd_lines")
+        if v is not None:
+            return int(v) % 128, int(v) // 128
+        n = max(self.Nx, self.Ny)
+        wgs = -(-kn // 32) * tab["sweep_grp_p"].shape[0]
+        nsplit = 1 if wgs >= 256 else max(1, min((512 + wgs // 2) // wgs, n // 8, 12))
+        return nsplit, int(n <= 128)
+
+    def _lines_part(self, tab, n_angles, kn):
+        """Floats of the line sweep's partial sinograms, the most any subset needs (so that the workspace does not
+        grow between the subsets of a run, whose steps may have been captured)."""
+        key = (getattr(self, "_subsets_version", 0), self.radon_variant.get("fwd_lines"), n_angles, kn)
+        cap = self._lines_caps.get(key)
+        if cap is None:
+            sets = [(tab, n_angles)]
+            if self.omega_subsets is not None and self._sub_tables is not None:
+                sets += [(t, len(s)) for t, s in zip(self._sub_tables, self.omega_subsets)]
+            cap = max(self._lines_variant(t, kn)[0] * n * self.My * kn for t, n in sets)
+            self._lines_caps = {**self._lines_caps, key: cap} if len(self._lines_caps) < 64 else {key: cap}
+        return cap
+
     def _bwd_variant(self, tab, kn):
         """The table backprojection's variant for kn orientation columns: radon_variant["bwd"] if set (by hand or by
         autotune), else by size. From 32 tiles of 8 x 8 pixels on the matrix-core form (us, SPDHG update, against the
@@ -1116,27 +1157,25 @@ class SinglePhaseForwardOperator:
         if tab is not None:
             cands = {}
             sl = _lib.load().dfm_radon_sweep_lines(self.Nx, self.Ny)
+            if tab["pairs_ok"] and max(self.Nx, self.Ny) <= 256:
+                # the line sweep first: the fastest at every measured configuration but small images
+                rv["fwd_lines"] = None
+                nsplit, _ = self._lines_variant(tab, kn)
+                cands.update({f"lines:{n}" + "+dup" * d: ("lines", n + 128 * d) for n in sorted({nsplit, 1})
+                              for d in (1, 0)})
             if sl and self.My <= 1024:         # 1024 rays per workgroup (512 for the 64-orientation form)
-                cands.update({f"sweep:{n}": ("sweep", n) for n in (8, 4, 2) if n <= sl})
+                cands.update({f"sweep:{n}": ("sweep", n) for n in (4,) if n <= sl})
                 ln = max(self.Nx, self.Ny)
                 for n in (2, 1):                 # 32 orientations per workgroup
                     if 2 * n * ln * 9 * 16 <= 163840:
                         cands[f"sweep:{n}+ch32"] = ("sweep", n + 16)
-            if tab["pairs_ok"]:
-                ln = max(self.Nx, self.Ny)
-                # first the duplicated-pixel layout (conflict-free LDS reads, twice the LDS: the fastest where it
-                # fits), then the plain layout, then the forms that load each staged block at its start (at most 128
-                # VGPRs: two workgroups per CU)
-                cands.update({f"psweep:{n}+dup": ("psweep", n + 16) for n in (2, 1)
-                              if (n == 1 or ln <= 128) and 2 * n * (ln + 5) * 256 <= 163840})
-                cands.update({f"psweep:{n}": ("psweep", n) for n in (2, 1, 4)
-                              if 2 * n * (ln + 4) * 128 <= 163840 and (n < 4 or ln <= 128)})
-                cands.update({f"psweep:{n}+np": ("psweep", n + 8) for n in (2, 1) if n == 1 or ln <= 128})
+            ln = max(self.Nx, self.Ny)
+            if tab["pairs_ok"] and ln <= 256:
+                # the register-staged ray pairs
+                cands.update({f"psweep:{n}": ("psweep", n) for n in (2, 1) if 2 * n * (ln + 4) * 128 <= 163840})
             if self.radon_bands > 1:
-                cands.update({"band:8+ch128": ("band", 8 + 16), "band:8": ("band", 8), "band:4": ("band", 4),
-                              "band:8+ch256": ("band", 8 + 32)})
-            cands.update({"table:8+lds+ch128": ("table", 8 + 256 + 1536), "table:8+lds": ("table", 8 + 256),
-                          "table:4+lds": ("table", 4 + 256)})
+                cands.update({"band:8+ch128": ("band", 8 + 16), "band:8": ("band", 8)})
+            cands.update({"table:8+lds+ch128": ("table", 8 + 256 + 1536), "table:8+lds": ("table", 8 + 256)})
             times = {}
             for name, (kern, v) in cands.items():
                 rv["fwd_kernel"] = kern
@@ -1148,6 +1187,8 @@ class SinglePhaseForwardOperator:
                     rv["fwd_sweep"] = v
                 elif kern == "psweep":
                     rv["fwd_psweep"] = v
+                elif kern == "lines":
+                    rv["fwd_lines"] = v
                 times[name] = timeit(lambda: self._radon_forward(img, img_kstride, koff, kn, sino, geo_f, n_ang, tab))
             best = _pick(times)
             kern, v = cands[best]
@@ -1160,6 +1201,8 @@ class SinglePhaseForwardOperator:
                 saved["fwd_sweep"] = v
             elif kern == "psweep":
                 saved["fwd_psweep"] = v
+            elif kern == "lines":
+                saved["fwd_lines"] = v
             out["radon_forward"] = (best, times)
             # the matrix-core form first (the fastest at every measured configuration but the smallest; the first listed
             # within the tolerance wins), then the 8x8-tile and the 4x4-tile forms
@@ -1168,8 +1211,8 @@ class SinglePhaseForwardOperator:
                 cands["mfma"] = ("table", BWD_MFMA)
             if tab["tbase8"].numel() > 1:
                 cands.update({f"table8:{a}x{g}": ("table", a + 64 * g + 1024)
-                              for a, g in ((8, 2), (8, 4), (8, 1), (4, 2), (4, 4), (4, 1))})
-            cands.update({f"table:{a}x{g}": ("table", a + 64 * g) for a, g in ((4, 4), (4, 2), (8, 4), (8, 2), (8, 8))})
+                              for a, g in ((8, 2), (8, 4), (8, 1))})
+            cands.update({f"table:{a}x{g}": ("table", a + 64 * g) for a, g in ((4, 4), (8, 2))})
             times = {}
             for name, (kern, v) in cands.items():
                 rv["bwd_kernel"] = kern
@@ -1317,27 +1360,36 @@ class SinglePhaseForwardOperator:
             with torch.cuda.stream(q):
                 self.fourier.forward(img, img_kstride, koff, kn, sino, self._fourier_angles(geo), self._stream())
             return
-        if tab is not None and self.radon_variant["fwd_kernel"] == "psweep" and tab["pairs_ok"]:
+        kernel = self.radon_variant["fwd_kernel"] or self._fwd_kernel(tab, n_angles, kn)
+        if tab is not None and kernel == "lines" and tab["pairs_ok"]:
+            nsplit, dup = self._lines_variant(tab, kn)
+            g = tab["sweep_grp_p"]
+            part = self._t_buf(self._lines_part(tab, n_angles, kn))[0] if nsplit > 1 else None
+            _lib.call("dfm_radon_forward_lines", _lib.ptr(img), _lib.ptr(sino), _lib.ptr(part),
+                      _lib.ptr(tab["sweep_geo"]), _lib.ptr(g), _lib.ptr(tab["sweep_gcls_p"]), g.shape[0], g.shape[1],
+                      n_angles, self.My, self.Nx, self.Ny, img_kstride, koff, kn, kn, nsplit, dup, self._stream())
+            return
+        if tab is not None and kernel == "psweep" and tab["pairs_ok"]:
             g = tab["sweep_grp_p"]
             _lib.call("dfm_radon_forward_pairs_sweep", _lib.ptr(img), _lib.ptr(sino), _lib.ptr(tab["sweep_geo"]),
                       _lib.ptr(g), _lib.ptr(tab["sweep_gcls_p"]), g.shape[0], g.shape[1], self.My, self.Nx, self.Ny,
                       img_kstride, koff, kn, kn, int(self.radon_variant.get("fwd_psweep", 2)), self._stream())
             return
-        if tab is not None and self.radon_variant["fwd_kernel"] in ("sweep", "psweep"):
+        if tab is not None and kernel in ("sweep", "psweep", "lines"):
             lines = self.radon_variant.get("fwd_sweep", 0) or _lib.load().dfm_radon_sweep_lines(self.Nx, self.Ny)
             g = tab["sweep_grp"]
             _lib.call("dfm_radon_forward_sweep", _lib.ptr(img), _lib.ptr(sino), _lib.ptr(tab["sweep_geo"]),
                       _lib.ptr(g), _lib.ptr(tab["sweep_gcls"]), g.shape[0], g.shape[1], self.My, self.Nx,
                       self.Ny, img_kstride, koff, kn, kn, int(lines), self._stream())
             return
-        if tab is not None and self.radon_variant["fwd_kernel"] == "band":
+        if tab is not None and kernel == "band":
             nb = self.radon_bands
             part = self._t_buf(nb * n_angles * self.My * kn)[0]
             _lib.call("dfm_radon_forward_band", _lib.ptr(img), _lib.ptr(sino), _lib.ptr(part),
                       _lib.ptr(tab["band_ptr"]), _lib.ptr(tab["pix"]), _lib.ptr(tab["w"]), self.My, n_angles, nb,
                       img_kstride, koff, kn, kn, self.radon_variant.get("fwd_band", 8), self._stream())
             return
-        if tab is not None and self.radon_variant["fwd_kernel"] != "arith":
+        if tab is not None and kernel != "arith":
             _lib.call("dfm_radon_forward_table", _lib.ptr(img), _lib.ptr(sino), _lib.ptr(tab["row_ptr"]),
                       _lib.ptr(tab["pix"]), _lib.ptr(tab["w"]), self.My, n_angles, img_kstride, koff, kn, kn,
                       self.radon_variant["fwd"], self._stream())

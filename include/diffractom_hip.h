@@ -113,6 +113,15 @@ int dfm_radon_forward_pairs_sweep(const float* img_k, float* sino, const double*
                                   const int32_t* grp_cls, int32_t n_grp, int32_t na_grp, int32_t ns, int32_t nx,
                                   int32_t ny, int32_t kstride, int32_t k_off, int32_t k_n, int32_t skstride,
                                   int32_t lines, dfm_stream_t stream);
+/* The same sums with every line brought into LDS by the load unit while the one before is summed; the lines may be
+ * split into nsplit ranges (1 to 64), each summed into a partial sinogram of part (nsplit * n_angles * ns * skstride
+ * floats; unused for nsplit 1) and added in order. dup: every pixel twice in LDS (no bank conflicts). Groups as for
+ * dfm_radon_forward_pairs_sweep, covering n_angles angles. An infinite or NaN pixel reaches only the rays that have a
+ * weight on it. */
+int dfm_radon_forward_lines(const float* img_k, float* sino, float* part, const double* geo, const int32_t* grp_ang,
+                            const int32_t* grp_cls, int32_t n_grp, int32_t na_grp, int32_t n_angles, int32_t ns,
+                            int32_t nx, int32_t ny, int32_t kstride, int32_t k_off, int32_t k_n, int32_t skstride,
+                            int32_t nsplit, int32_t dup, dfm_stream_t stream);
 /* The forward projection of dfm_radon_forward_table tiled by nb bands of image rows: band_ptr[(a ns + s) nb + b]
  * is the first table entry of ray (a, s) in band b (entries ascend in pixel index), band_ptr[na ns nb] the total.
  * Per band the partial sums go to part (nb * n_angles * ns * skstride floats), then sino = their sum in band order.
