@@ -53,7 +53,17 @@ class _BlkDesc(ctypes.Structure):
 def _y_tiling(my):
     tiles = -(-my // 16)
     n_yg = -(-tiles // 8)
-    return -(-tiles // n_yg), n_yg
+    mt_n = -(-tiles // n_yg)
+    return mt_n, n_yg
+
+
+def _blk_y_tiling(my, stride):
+    """y tiles per group and y groups of the block-sparse products (y_tiling of csrc/pf_blocks.hip): 1 and 3 tiles run
+    as 2 and 4 (the counts with a compiled form); a group's rows stay below 4 GiB."""
+    mt_n, n_yg = _y_tiling(my)
+    if stride >= 1 << 23:
+        return 2, -(-my // 32)
+    return mt_n + (mt_n in (1, 3)), n_yg
 
 
 class BatchedSPDHGPoisson:
@@ -177,9 +187,9 @@ class BatchedSPDHGPoisson:
         o0 = self.ops[0]
         R, My, CP = o0.N_Omega, o0.My, o0.N_seg
         n_ang = R if m is None else len(self.subsets[m])
-        mt_n, n_yg = _y_tiling(My)
         if self.blocks:
-            return self._blk_group(forward, m, key, n_ang, mt_n, n_yg)
+            return self._blk_group(forward, m, key, n_ang, *_blk_y_tiling(My, self.Kc))
+        mt_n, n_yg = _y_tiling(My)
         descs = (_Desc * len(self.ops))()
         wg = []
         for i, op in enumerate(self.ops):
@@ -268,7 +278,7 @@ class BatchedSPDHGPoisson:
         buf, wgm, n_wg = self._group(forward, m)
         if self.blocks:
             # + the slices' common y-tile count in bits 8-11 (a compiled form where there is one; same results)
-            mt_n, _ = _y_tiling(self.ops[0].My)
+            mt_n, _ = _blk_y_tiling(self.ops[0].My, self.Kc)
             _lib.call("dfm_pfblk_grouped", int(forward), _lib.ptr(buf), _lib.ptr(wgm), n_wg,
                       (self.ops[0]._blk_mode("fwd") & 15) | (mt_n << 8), self.ops[0]._stream())
             return

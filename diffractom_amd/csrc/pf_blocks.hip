@@ -16,7 +16,11 @@
 // 32. Per chunk it expands its block into dense MFMA fragments in a private LDS area (clear, scatter the block's
 // entries, read back in operand order: lane l holds 8 consecutive contraction indices of column l % 16), while the
 // workgroup's four waves share the y-side operand chunk (FP32 from HBM, split into bf16 hi/lo or scaled to fp16 in
-// LDS, double buffered). v_mfma_f32_16x16x32_{bf16,f16}, FP32 accumulation; the residual mode adds hi*hi + hi*lo +
+// LDS, double buffered). What bounds it: the chunk's latency (loads, LDS expansion, barrier), so the loads run two
+// chunks ahead, in code without branches around them, and the tile loops have compiled counts. 18 angles x 103 rows x
+// 29,713 orientations x 1,440 segments (65 GFLOP of tiles, 0.28 GB of PF), loads in branches / as here: residual
+// forward 511 / 387 us, adjoint 389 / 341; fp16 557 / 411 and 445 / 430; 90 angles x 131 rows x 5,000 x 1,440,
+// residual: 722 / 520 and 557 / 459. v_mfma_f32_16x16x32_{bf16,f16}, FP32 accumulation; the residual mode adds hi*hi + hi*lo +
 // lo*hi (lo*lo, 2^-16 relative, dropped). In the fp16 mode every (row, chunk) of the y-side operand is scaled by a
 // power of two that puts its largest magnitude at 2^14 (fp16 keeps 11 significant bits from 2^-14 up), and the
 // product of the chunk is scaled back before it is added to the FP32 accumulator; the ring scale of the PF is
@@ -158,14 +162,20 @@ __device__ __forceinline__ void blk_pf_body(const BlkArgs& p, int64_t w) {
   constexpr bool RES = MODE == MODE_BF16_RES;
   constexpr bool F16 = MODE == MODE_F16;
   constexpr int TH = 64 * WV;                                // threads of the workgroup
+  constexpr int MTB = MTN > 0 && MTN * 64 <= TH ? TH / 64 : MT_MAX;  // y tiles staged: whole passes of the workgroup
   // y-side operand, double buffered: fragment s = mt * 64 + lane (8 consecutive contraction indices of a row)
-  __shared__ s16x8 a_hi[2 * MT_MAX * 64];
-  __shared__ s16x8 a_lo[RES ? 2 * MT_MAX * 64 : 1];
-  __shared__ __align__(16) float a_inv[F16 ? 2 * MT_MAX * 16 : 4];   // fp16 mode: 1 / scale of each chunk row
+  __shared__ s16x8 a_hi[2 * MTB * 64];
+  __shared__ s16x8 a_lo[RES ? 2 * MTB * 64 : 1];
+  __shared__ __align__(16) float a_inv[F16 ? 2 * MTB * 16 : 4];   // fp16 mode: 1 / scale of each chunk row
   // each wave's expanded PF block: [hi / lo][tile][lane] fragments
   __shared__ s16x8 b_frag[WV][RES ? 2 : 1][2][64];
 
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  // fp16 adjoint: 1 / ring scale, folded into the staged data (read from memory where there are more rings)
+  constexpr int RING_LDS = 32;
+  __shared__ float ring_l[F16 && !FWD ? RING_LDS : 1];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int tg = (int)(w % p.n_tg);
   w /= p.n_tg;
   const int yg = (int)(w % p.n_yg);
@@ -183,52 +193,78 @@ __device__ __forceinline__ void blk_pf_body(const BlkArgs& p, int64_t w) {
   const int c0 = ks * p.ch_per;
   const int c1 = min(p.n_ch, c0 + p.ch_per);
   if (c0 >= c1) return;                                      // uniform
+  if (F16 && !FWD)
+    if (tid < min(p.P, RING_LDS)) ring_l[tid] = p.ring_inv[tid];
 
-  // ---- y-side operand slots of this thread: s = tid + TH i < mt_n * 64
-  const int n_slots = mt_n * 64;
-  constexpr int NS = (MT_MAX * 64 + TH - 1) / TH;
-  const float* srow[NS];
-  bool sok[NS];
-  const int64_t src_rows = FWD ? (int64_t)a * p.my : (int64_t)r * p.my;
+  // The loads of the pipeline below are issued without branches (clamped addresses instead): around a load that may not
+  // have been issued the compiler cannot count the ones in flight, and waits for all of them at every chunk.
+
+  // ---- y-side operand slots of this thread: s = tid + TH i, all MTB tiles; rows beyond the group's last repeat it
+  // (their products go to no output)
+  constexpr int NS = MTB * 64 / TH;
+  const int64_t src_rows = (FWD ? (int64_t)a * p.my : (int64_t)r * p.my) + y0;
+  const int rows = min(p.my - y0, mt_n * 16);
   const int src_stride = FWD ? p.sks : p.cp;
   const int src_n = FWD ? p.kb : p.cp;
-  const bool vec = (src_stride & 3) == 0;
+  const int c_full = src_n >> 5;                             // chunks with all 32 columns; at most one after them
+  const int scol = ((tid & 63) >> 4) * 8;                    // the same for every slot of this thread
+  // the group's rows as a buffer (reads past its end give 0; they occur where there are fewer than 32 columns in all),
+  // and this thread's byte offsets in it
+  const float* src = p.src + src_rows * src_stride;
+  const __amdgpu_buffer_rsrc_t rsrc =
+      __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, (unsigned)rows * (unsigned)src_stride * 4u, 0x00027000);
+  unsigned soff[NS];
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
     const int s = tid + TH * i;
-    const int y = y0 + (s >> 6) * 16 + (s & 15);
-    sok[i] = s < n_slots && y < p.my;
-    srow[i] = p.src + (src_rows + (sok[i] ? y : 0)) * src_stride;
+    const int y = min((s >> 6) * 16 + (s & 15), rows - 1);
+    soff[i] = ((unsigned)y * (unsigned)src_stride + scol) * 4u;
   }
-  const int scol = ((tid & 63) >> 4) * 8;                    // the same for every slot of this thread
-  // the ring of column j (adjoint fp16 mode): (c * 32 + scol) % P once per chunk, then stepped
+  typedef unsigned u4 __attribute__((ext_vector_type(4)));
+  // the rows of a full chunk (chunks beyond the range, or the last one with fewer columns, repeat the last full one)
   auto load_raw = [&](int c, float (&raw)[NS][8]) {
-    const int j0 = c * 32 + scol;
-    int jr = 0;
-    if (F16 && !FWD) jr = j0 % p.P;
+    const int cbyte = max(min(min(c, c1 - 1), c_full - 1), 0) * 128;
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
-      if (sok[i] && vec && j0 + 8 <= src_n) {
-        const float4 u = *reinterpret_cast<const float4*>(srow[i] + j0);
-        const float4 v = *reinterpret_cast<const float4*>(srow[i] + j0 + 4);
-        raw[i][0] = u.x; raw[i][1] = u.y; raw[i][2] = u.z; raw[i][3] = u.w;
-        raw[i][4] = v.x; raw[i][5] = v.y; raw[i][6] = v.z; raw[i][7] = v.w;
-      } else {
+      const u4 u = __builtin_amdgcn_raw_buffer_load_b128(rsrc, soff[i], cbyte, 0);
+      const u4 v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, soff[i] + 16, cbyte, 0);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) raw[i][e] = (sok[i] && j0 + e < src_n) ? srow[i][j0 + e] : 0.f;
-      }
-      if (F16 && !FWD) {
-        // the ring scale of the PF folded into the data: column j = j0 + e, ring j % P
-        int q = jr;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          raw[i][e] *= p.ring_inv[q];
-          q = q + 1 == p.P ? 0 : q + 1;
-        }
+      for (int e = 0; e < 4; ++e) {
+        raw[i][e] = __builtin_bit_cast(float, (unsigned)u[e]);
+        raw[i][4 + e] = __builtin_bit_cast(float, (unsigned)v[e]);
       }
     }
   };
-  auto store_lds = [&](int buf, float (&raw)[NS][8]) {
+  // waits, in straight-line code, for the loads that made v: a load that a branch skips stays in flight for the compiler,
+  // which then waits for everything where the register is next written
+  auto arrived = [](auto& v) { asm volatile("" : "+v"(v)); };
+  auto store_lds = [&](int c, int buf, float (&raw)[NS][8]) {
+    const int j0 = c * 32 + scol;
+#pragma unroll
+    for (int i = 0; i < NS; ++i)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) arrived(raw[i][e]);
+    if (c >= c_full) {                                       // uniform: the chunk with fewer columns
+#pragma unroll
+      for (int i = 0; i < NS; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) raw[i][e] = j0 + e < src_n ? src[(soff[i] >> 2) + c * 32 + e] : 0.f;
+#pragma unroll
+      for (int i = 0; i < NS; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) arrived(raw[i][e]);
+    }
+    if (F16 && !FWD) {
+      // the ring scale of the PF folded into the data: column j = j0 + e, ring j % P
+      int q = j0 % p.P;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float f = q < RING_LDS ? ring_l[q] : p.ring_inv[q];
+#pragma unroll
+        for (int i = 0; i < NS; ++i) raw[i][e] *= f;
+        q = q + 1 == p.P ? 0 : q + 1;
+      }
+    }
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
       const int s = tid + TH * i;
@@ -245,11 +281,9 @@ __device__ __forceinline__ void blk_pf_body(const BlkArgs& p, int64_t w) {
         s16x8 h;
 #pragma unroll
         for (int e = 0; e < 8; ++e) h[e] = (short)f16_bits(raw[i][e] * sc);
-        if (s < n_slots) {
-          a_hi[buf * MT_MAX * 64 + s] = h;
-          if ((s & 63) < 16) a_inv[buf * MT_MAX * 16 + (s >> 6) * 16 + (s & 15)] = 1.f / sc;
-        }
-      } else if (s < n_slots) {
+        a_hi[buf * MTB * 64 + s] = h;
+        if ((s & 63) < 16) a_inv[buf * MTB * 16 + (s >> 6) * 16 + (s & 15)] = 1.f / sc;
+      } else {
         s16x8 h, l;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -257,18 +291,19 @@ __device__ __forceinline__ void blk_pf_body(const BlkArgs& p, int64_t w) {
           h[e] = (short)__builtin_bit_cast(unsigned short, hb);
           if (RES) l[e] = (short)bf16_bits(raw[i][e] - (float)hb);
         }
-        a_hi[buf * MT_MAX * 64 + s] = h;
-        if (RES) a_lo[buf * MT_MAX * 64 + s] = l;
+        a_hi[buf * MTB * 64 + s] = h;
+        if (RES) a_lo[buf * MTB * 64 + s] = l;
       }
     }
   };
 
   // ---- this wave's PF blocks: block (r, kb, jb) with kb = chunk (forward) or the column block (adjoint)
+  const bool have = cb_live && cb_stored;
+  const int cbx = have ? cb : 0;
   auto blk_index = [&](int c) -> int64_t {
-    const int kbi = FWD ? c : cb, jbi = FWD ? cb : c;
+    const int kbi = FWD ? c : cbx, jbi = FWD ? cbx : c;
     return ((int64_t)(p.blk_local ? a : r) * p.n_kb + kbi) * p.n_jb + jbi;
   };
-  const bool have = cb_live && cb_stored;
   const unsigned* v32 = (const unsigned*)p.val;
   const unsigned short* v16 = (const unsigned short*)p.val;
   // the entries of chunk c's block: its range [lo, hi) and the first ER * 64 (ER per lane), fetched two chunks ahead
@@ -276,28 +311,23 @@ __device__ __forceinline__ void blk_pf_body(const BlkArgs& p, int64_t w) {
   constexpr int ER = 4;
   struct Ent {
     int lo, hi;
+    bool live;                                               // a chunk of the range
     unsigned pp[ER], vv[ER];
   };
-  // the block range of chunk c (two dependent loads: the pointers are fetched one chunk before the entries, so that
-  // the wait for them never includes the loads issued in the same chunk)
-  auto fetch_ptr = [&](int c, int2& q) {
-    q = make_int2(0, 0);
-    if (have && c < c1) {
-      const int64_t bi = blk_index(c);
-      q.x = p.ptr[bi];
-      q.y = p.ptr[bi + 1];
-    }
-  };
-  auto fetch = [&](const int2& q, Ent& E) {
-    E.lo = q.x;
-    E.hi = q.y;
+  // the block range of chunk c, in lanes 0 and 1 (a vector load: scalar ones would be waited for with every LDS read),
+  // one chunk before the entries that need it
+  auto fetch_ptr = [&](int c, int& q) { q = p.ptr[blk_index(min(c, c1 - 1)) + (lane & 1)]; };
+  auto fetch = [&](int c, int q, Ent& E) {
+    const int lo = __builtin_amdgcn_readlane(q, 0), hi = __builtin_amdgcn_readlane(q, 1);
+    E.lo = lo;
+    E.hi = have && c < c1 ? hi : lo;
+    E.live = have && c < c1;
+    const int last = max(hi - 1, 0);
 #pragma unroll
     for (int u = 0; u < ER; ++u) {
-      const int e = E.lo + 64 * u + lane;
-      if (e < E.hi) {
-        E.pp[u] = p.pos[e];
-        E.vv[u] = F16 ? (unsigned)v16[e] : v32[e];
-      }
+      const int e = min(lo + 64 * u + lane, last);
+      E.pp[u] = p.pos[e];
+      E.vv[u] = F16 ? (unsigned)v16[e] : v32[e];
     }
   };
   short* bf = reinterpret_cast<short*>(&b_frag[wv][0][0][0]);   // the element type of the s16x8 fragments
@@ -314,8 +344,13 @@ __device__ __forceinline__ void blk_pf_body(const BlkArgs& p, int64_t w) {
 
   // chunk c: expand its block into the wave's fragments (in-order LDS accesses of one wave: the clear, the scatter
   // and the read-back need no barrier) and multiply with the y-side operand in LDS buffer buf
-  auto compute = [&](int buf, const Ent& E) {
-    if (!have) return;
+  auto compute = [&](int buf, Ent& E) {
+#pragma unroll
+    for (int u = 0; u < ER; ++u) {
+      arrived(E.pp[u]);
+      arrived(E.vv[u]);
+    }
+    if (!E.live) return;                                     // uniform
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       b_frag[wv][0][t][lane] = zero8;
@@ -338,9 +373,9 @@ __device__ __forceinline__ void blk_pf_body(const BlkArgs& p, int64_t w) {
 #pragma unroll
     for (int mt = 0; mt < MT_MAX; ++mt) {
       if (mt < mt_n) {
-        const s16x8 ah = a_hi[buf * MT_MAX * 64 + mt * 64 + lane];
+        const s16x8 ah = a_hi[buf * MTB * 64 + mt * 64 + lane];
         if (F16) {
-          const float4 iv = *reinterpret_cast<const float4*>(&a_inv[buf * MT_MAX * 16 + mt * 16 + (lane >> 4) * 4]);
+          const float4 iv = *reinterpret_cast<const float4*>(&a_inv[buf * MTB * 16 + mt * 16 + (lane >> 4) * 4]);
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
             const f32x4 d = mma_f16(ah, bh[t], f32x4{0.f, 0.f, 0.f, 0.f});
@@ -351,7 +386,7 @@ __device__ __forceinline__ void blk_pf_body(const BlkArgs& p, int64_t w) {
           }
           __builtin_amdgcn_sched_barrier(0);   // one row tile's products at a time (register pressure)
         } else {
-          const s16x8 al = RES ? a_lo[buf * MT_MAX * 64 + mt * 64 + lane] : zero8;
+          const s16x8 al = RES ? a_lo[buf * MTB * 64 + mt * 64 + lane] : zero8;
 #pragma unroll
           for (int t = 0; t < 2; ++t) {
             acc[mt][t] = mma_bf16(ah, bh[t], acc[mt][t]);
@@ -371,29 +406,36 @@ __device__ __forceinline__ void blk_pf_body(const BlkArgs& p, int64_t w) {
   // The loop is unrolled by two so that the register sets alternate roles instead of being copied.
   float rawA[NS][8], rawB[NS][8];
   Ent E0, E1;
-  int2 Q0, Q1;                                               // block ranges of chunks c + 2 and c + 3
+  int Q0, Q1;                                                // block ranges of chunks c + 2 and c + 3
+  if (F16 && !FWD) __syncthreads();                          // ring_l
   load_raw(c0, rawA);
-  store_lds(0, rawA);
-  if (c0 + 1 < c1) load_raw(c0 + 1, rawA);
+  store_lds(c0, 0, rawA);
+  load_raw(c0 + 1, rawA);
   fetch_ptr(c0, Q0);
   fetch_ptr(c0 + 1, Q1);
-  fetch(Q0, E0);
-  fetch(Q1, E1);
-  fetch_ptr(c0 + 2, Q0);
+  int Q2;
+  fetch_ptr(c0 + 2, Q2);
+  // in this order: the loop's waits also hold for its first pass
+  __builtin_amdgcn_sched_barrier(0);
+  fetch(c0, Q0, E0);
+  __builtin_amdgcn_sched_barrier(0);
+  fetch(c0 + 1, Q1, E1);
+  __builtin_amdgcn_sched_barrier(0);
+  Q0 = Q2;
   __syncthreads();
   // chunk c: the ranges of chunk c + 3 into qn, the rows of chunk c + 2, compute chunk c, the entries of chunk
   // c + 2 (range qe, fetched one chunk ago), the rows of chunk c + 1 to the other LDS buffer
-  auto step = [&](int c, int buf, float (&rin)[NS][8], float (&rout)[NS][8], Ent& E, const int2& qe, int2& qn) {
+  auto step = [&](int c, int buf, float (&rin)[NS][8], float (&rout)[NS][8], Ent& E, const int& qe, int& qn) {
     fetch_ptr(c + 3, qn);
-    if (c + 2 < c1) load_raw(c + 2, rout);
+    load_raw(c + 2, rout);
     compute(buf, E);
-    fetch(qe, E);
-    if (c + 1 < c1) store_lds(buf ^ 1, rin);
+    fetch(c + 2, qe, E);
+    store_lds(min(c + 1, c1 - 1), buf ^ 1, rin);             // (after the last chunk: nobody reads it)
     __syncthreads();
   };
   for (int c = c0; c < c1; c += 2) {
     step(c, 0, rawA, rawB, E0, Q0, Q1);
-    if (c + 1 < c1) step(c + 1, 1, rawB, rawA, E1, Q1, Q0);
+    step(c + 1, 1, rawB, rawA, E1, Q1, Q0);                  // (beyond the last chunk: nothing to compute)
   }
 
   if (!cb_live) return;
@@ -436,15 +478,12 @@ __global__ __launch_bounds__(64 * WV, WV == 4 ? (MODE == MODE_F16 ? 2 : 3) : 2) 
   blk_pf_body<MODE, FWD, WV, MTN>(p, xcd_block());
 }
 
-// the y-tile counts compiled in (MTN) for the 4-wave form: 7 (97-112 detector rows in one group) and 6 (groups of
-// 6 tiles, e.g. 261 rows in three)
-
 // Grouped launch: workgroup w runs workgroup wg_map[w].y of product wg_map[w].x (the slices of a multi-slice batch,
 // each its own PF blocks, K, sinogram columns and data rows); entries with x < 0 pad the grid.
 // (MTN > 0: every descriptor's y-tile count, compiled in)
 template <int MODE, bool FWD, int MTN>
-__global__ __launch_bounds__(THREADS, MODE == MODE_F16 ? 2 : 3) void blk_pf_grouped_kernel(const BlkArgs* __restrict__ descs,
-                                                                    const int2* __restrict__ wg_map, int64_t n_map) {
+__global__ __launch_bounds__(THREADS, MODE == MODE_F16 || MTN == 0 ? 2 : 3) void blk_pf_grouped_kernel(
+    const BlkArgs* __restrict__ descs, const int2* __restrict__ wg_map, int64_t n_map) {
   const int64_t w = xcd_block();
   if (w >= n_map) return;
   const int2 m = wg_map[w];
@@ -464,12 +503,6 @@ void launch_blk_grouped_mt(const BlkArgs* descs, const int2* wg_map, int64_t n_m
     hipLaunchKernelGGL((blk_pf_grouped_kernel<MODE_F16, FWD, MTN>), grid, block, 0, st, descs, wg_map, n_map);
 }
 
-template <bool FWD>
-void launch_blk_grouped(const BlkArgs* descs, const int2* wg_map, int64_t n_map, int mode, int mtn, hipStream_t st) {
-  if (mtn == 5) launch_blk_grouped_mt<FWD, 5>(descs, wg_map, n_map, mode, st);
-  else launch_blk_grouped_mt<FWD, 0>(descs, wg_map, n_map, mode, st);
-}
-
 template <bool FWD, int WV, int MTN>
 void launch_blk_wv(const BlkArgs& p, int mode, hipStream_t st) {
   const int64_t n_wg = (int64_t)p.n_ang * p.ksplit * p.n_yg * p.n_tg;
@@ -479,22 +512,53 @@ void launch_blk_wv(const BlkArgs& p, int mode, hipStream_t st) {
   else hipLaunchKernelGGL((blk_pf_kernel<MODE_F16, FWD, WV, MTN>), grid, block, 0, st, p);
 }
 
+// y tiles per group that have a 4-wave form with the count compiled in: the tile loops carry no run-time bound, so a
+// chunk's LDS reads and MFMAs are one straight block, and three workgroups fit a CU (residual, 7 tiles: 184 VGPRs with
+// the run-time count, 168 compiled). Other counts run as the next larger one or, grouped, in the run-time form.
+#define DFM_MT(MT, CALL)                                                                                           \
+  switch (MT) {                                                                                                    \
+    case 2: { constexpr int N = 2; CALL; break; }                                                                  \
+    case 4: { constexpr int N = 4; CALL; break; }                                                                  \
+    case 5: { constexpr int N = 5; CALL; break; }                                                                  \
+    case 6: { constexpr int N = 6; CALL; break; }                                                                  \
+    case 7: { constexpr int N = 7; CALL; break; }                                                                  \
+    default: { constexpr int N = 8; CALL; }                                                                        \
+  }
+
 template <bool FWD>
-void launch_blk(const BlkArgs& p, int mode, int wv, bool fixed, hipStream_t st) {
-  if (wv == 8) launch_blk_wv<FWD, 8, 0>(p, mode, st);
-  else if (fixed && p.mt_n == 7) launch_blk_wv<FWD, 4, 7>(p, mode, st);
-  else if (fixed && p.mt_n == 6) launch_blk_wv<FWD, 4, 6>(p, mode, st);
-  else launch_blk_wv<FWD, 4, 0>(p, mode, st);
+void launch_blk_grouped(const BlkArgs* descs, const int2* wg_map, int64_t n_map, int mode, int mtn, hipStream_t st) {
+  if (mtn == 2 || (mtn >= 4 && mtn <= MT_MAX)) {
+    DFM_MT(mtn, (launch_blk_grouped_mt<FWD, N>(descs, wg_map, n_map, mode, st)))
+  } else {
+    launch_blk_grouped_mt<FWD, 0>(descs, wg_map, n_map, mode, st);
+  }
 }
 
-// waves per workgroup from bits 5-6 of the mode argument: 0 -> 4, 1 -> 8; bit 7: the 4-wave form with the y-tile
-// count compiled in where it is 6 or 7 (the same results)
+template <bool FWD>
+void launch_blk(const BlkArgs& p, int mode, int wv, hipStream_t st) {
+  if (wv == 8) {
+    launch_blk_wv<FWD, 8, 0>(p, mode, st);
+    return;
+  }
+  DFM_MT(p.mt_n, (launch_blk_wv<FWD, 4, N>(p, mode, st)))
+}
+#undef DFM_MT
+
+// waves per workgroup from bits 5-6 of the mode argument: 0 -> 4, 1 -> 8 (bit 7 is accepted and changes nothing)
 int mode_waves(int mode) { return 4 << ((mode >> 5) & 3); }
 
-void y_tiling(int my, int& mt_n, int& n_yg) {
+// y tiles per group and y groups; a group's source rows are one buffer of less than 4 GiB, so very long rows go in
+// groups of 32
+void y_tiling(int my, int stride, int& mt_n, int& n_yg) {
   const int tiles = (my + 15) / 16;
+  if (stride >= 1 << 23) {
+    mt_n = 2;
+    n_yg = (tiles + 1) / 2;
+    return;
+  }
   n_yg = (tiles + MT_MAX - 1) / MT_MAX;
   mt_n = (tiles + n_yg - 1) / n_yg;
+  mt_n += mt_n == 1 || mt_n == 3;                            // the next compiled count
 }
 
 }  // namespace
@@ -535,7 +599,6 @@ int dfm_pfblk_forward(const float* sino, int32_t sks, int32_t kb, const int32_t*
   const int local = (mode >> 4) & 1;
   const int wv = mode_waves(mode);
   DFM_CHECK_ARG(wv <= 8, "dfm_pfblk_forward: waves code %d (0, 1: 4, 8 waves per workgroup)", (mode >> 5) & 3);
-  const bool fixed = (mode >> 7) & 1;
   mode &= 15;
   DFM_CHECK_ARG(mode >= MODE_BF16 && mode <= MODE_F16 && (mode != MODE_F16 || (ring_inv && P > 0)),
                 "dfm_pfblk_forward: mode %d (0 bf16, 1 bf16 residual, 2 fp16 with ring scales)", mode);
@@ -561,7 +624,7 @@ int dfm_pfblk_forward(const float* sino, int32_t sks, int32_t kb, const int32_t*
   p.kb = kb;
   p.n_cb = p.n_jb;
   p.n_ch = p.n_kb;
-  y_tiling(my, p.mt_n, p.n_yg);
+  y_tiling(my, sks, p.mt_n, p.n_yg);
   p.n_tg = (p.n_cb + wv - 1) / wv;
   p.ch_per = (p.n_ch + ksplit - 1) / ksplit;
   p.ksplit = (p.n_ch + p.ch_per - 1) / p.ch_per;
@@ -570,7 +633,7 @@ int dfm_pfblk_forward(const float* sino, int32_t sks, int32_t kb, const int32_t*
   p.out = p.direct ? data : part;
   p.alpha = 1.f;
   const hipStream_t st = (hipStream_t)stream;
-  launch_blk<true>(p, mode, wv, fixed, st);
+  launch_blk<true>(p, mode, wv, st);
   DFM_LAUNCH_CHECK("dfm_pfblk_forward");
   if (!p.direct) return dfm::launch_splitk_reduce(part, data, omegas, n_ang, (int64_t)my * cp, p.ksplit, accumulate, st);
   return DFM_OK;
@@ -583,7 +646,6 @@ int dfm_pfblk_adjoint(const float* data, const int32_t* ptr, const uint16_t* pos
   const int local = (mode >> 4) & 1;
   const int wv = mode_waves(mode);
   DFM_CHECK_ARG(wv <= 8, "dfm_pfblk_adjoint: waves code %d (0, 1: 4, 8 waves per workgroup)", (mode >> 5) & 3);
-  const bool fixed = (mode >> 7) & 1;
   mode &= 15;
   DFM_CHECK_ARG(mode >= MODE_BF16 && mode <= MODE_F16 && (mode != MODE_F16 || (ring_inv && P > 0)),
                 "dfm_pfblk_adjoint: mode %d (0 bf16, 1 bf16 residual, 2 fp16 with ring scales)", mode);
@@ -608,13 +670,13 @@ int dfm_pfblk_adjoint(const float* data, const int32_t* ptr, const uint16_t* pos
   p.kb = sks;
   p.n_cb = (sks + 31) / 32;           // every sinogram column is written (those of no stored block with 0)
   p.n_ch = p.n_jb;
-  y_tiling(my, p.mt_n, p.n_yg);
+  y_tiling(my, cp, p.mt_n, p.n_yg);
   p.n_tg = (p.n_cb + wv - 1) / wv;
   p.ksplit = 1;
   p.ch_per = p.n_ch;
   p.alpha = alpha;
   p.ncols = sks;
-  launch_blk<false>(p, mode, wv, fixed, (hipStream_t)stream);
+  launch_blk<false>(p, mode, wv, (hipStream_t)stream);
   DFM_LAUNCH_CHECK("dfm_pfblk_adjoint");
   return DFM_OK;
 }
@@ -622,7 +684,8 @@ int dfm_pfblk_adjoint(const float* data, const int32_t* ptr, const uint16_t* pos
 int dfm_pfblk_grouped(int32_t forward, const void* descs, const int32_t* wg_map, int64_t n_wg, int32_t mode,
                       dfm_stream_t stream) {
   DFM_CHECK_ARG(descs && wg_map && n_wg > 0, "dfm_pfblk_grouped: null pointer or no workgroups");
-  // bits 8-11: every descriptor's y-tile count mt_n, when the caller knows it (5 has a compiled form; 0: unknown)
+  // bits 8-11: every descriptor's y-tile count mt_n, when the caller knows it (2 and 4 to 8 have a compiled form; 0:
+  // unknown)
   const int mtn = (mode >> 8) & 15;
   mode &= 15;
   DFM_CHECK_ARG(mode >= MODE_BF16 && mode <= MODE_F16, "dfm_pfblk_grouped: mode %d", mode);

@@ -286,7 +286,8 @@ int dfm_mfma_grouped(int32_t forward, const dfm_mfma_desc* descs, const int32_t*
  * k < sks (0 at and beyond kb). mode: 0 bf16 (val hi only), 1 bf16 with the hi/lo residual correction (hi*hi + hi*lo
  * + lo*hi), 2 fp16 (val fp16; ring_inv[p] = 1 / ring_scale[p]; the y-side operand scaled by a power of two per row
  * and chunk of 32); + 16: the blocks are indexed by the position a in the angle list (a generated PF of just these
- * angles, dfm_pfgen) instead of by omegas[a]. FP32 accumulation. */
+ * angles, dfm_pfgen) instead of by omegas[a]; + 32: 8 waves per workgroup; + 128: accepted, changes nothing. FP32
+ * accumulation. */
 int dfm_pfblk_count(const float* pf, int32_t* counts, int32_t R, int32_t km, int32_t kb, int32_t cp,
                     dfm_stream_t stream);
 int dfm_pfblk_fill(const float* pf, const int32_t* ptr, uint16_t* pos, void* val, int32_t fp16,
@@ -306,7 +307,7 @@ int dfm_pfblk_adjoint(const float* data, const int32_t* ptr, const uint16_t* pos
  * dfm_pfblk_adjoint: src the sinogram (forward, first column of the product) or the data; out the data (direct = 1)
  * or the partial sums (forward), the sinogram (adjoint); n_kb / n_jb the stored blocks; n_cb the output column
  * blocks of 32 (forward n_jb, adjoint ceil(sks / 32)) and n_ch the contraction chunks; mt_n, n_yg the y tiling
- * (n_yg = ceil(ceil(my / 16) / 8) groups of mt_n 16-row tiles); n_tg = ceil(n_cb / 4); ch_per chunks per split. */
+ * (n_yg groups of mt_n <= 8 16-row tiles, n_yg mt_n 16 >= my, a group's rows below 4 GiB); n_tg = ceil(n_cb / 4); ch_per chunks per split. */
 typedef struct dfm_pfblk_desc {
   const float* src;
   const int32_t* ptr;
