@@ -7,13 +7,18 @@
 // with r = omegas[a] the angle's data row (pf_kernels.cl:597-687 spmm_pf_forward_c / spmm_pf_adjoint_c;
 // single_phase_forward_operator.py:38-123).
 //
-// A workgroup of 16 waves owns 16 R consecutive CSR rows of one angle and one column range (split s). It walks the
-// range in chunks of kc columns: the chunk of `in` (kc rows of ys floats, contiguous) is staged in LDS, then every wave
-// consumes, for each of its R rows, the row's entries that fall in the chunk. The lanes of a wave run over the
-// detector positions y (YW groups of 64), so an entry is wave-uniform (its column read from the row's 64-entry window
-// held in registers with v_readlane, its value likewise from the window's values) and its operand is one
-// conflict-free LDS row read. Per row the column window moves on only when all 64 of its entries are consumed.
-// Summation follows the CSR order, as in the row-per-thread kernels.
+// A workgroup of 16 waves owns 64 R consecutive CSR rows of one angle and one column range (split s). It walks the
+// range in chunks of kc columns: the chunk of `in` (kc rows of ys floats) is staged in LDS, then every wave consumes, for
+// each of its R quads of rows, the rows' entries that fall in the chunk. A row belongs to 16 lanes (four rows at once in
+// a wave), each holding 4 detector positions of every 64: the 16 lanes hold a window of 16 entries of their row, entry t
+// reaches all of them as a DPP row broadcast (its value as an operand of the FMA, its LDS offset of the address add) and
+// its operand is one contiguous 16-byte read per lane. Four entries cost 1 add, 4 NB FMAs and NB LDS reads for 64 NB
+// detector positions; with an entry per wave-instruction (two v_readlane, an add and 4-byte reads each) they cost 4
+// times (3 + NB), and that issue rate bounded the kernel: 9899 orientations x 180 angles x 900 segments x 103 rows, 6.2 %
+// fill (9.9e7 entries), forward 2.59 -> 1.63 ms with its split and transposes, adjoint 1.32 ms. VALU issue (82 % of the
+// cycles) still bounds it: a third of it entries, the rest the visits, their rounding to 4 entries and the staging. Rows whose entries run out in a chunk before the others' of
+// their quad read a zero operand. The first two windows of a visit are loaded one visit ahead. Summation follows the CSR
+// order, as in the row-per-thread kernels.
 #include <algorithm>
 
 #include "dfm_common.h"
@@ -23,111 +28,185 @@ namespace {
 constexpr int SPT_WAVES = 16;
 constexpr int SPT_LDS_FLOATS = 40960;   // 160 KiB
 
-template <int R, int YW, int U>
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// lane K of every 16 lanes, to those 16 lanes (DPP row_newbcast)
+template <int K>
+__device__ __forceinline__ int bcast16(int x) {
+  return __builtin_amdgcn_update_dpp(0, x, 0x150 + K, 0xf, 0xf, true);
+}
+
+// An operand row in LDS is NB blocks of 16 units of 16 bytes; unit u of row c lies at u ^ swz(c) of its block. Rows of
+// whole blocks: the 16-byte reads of a wave go 16 lanes at a time, 8 of one window's 16 lanes (0-3 and 12-15, or 4-11) and
+// the other 8 positions of another's, so rows at one bank offset, whatever they are, never conflict (with rows of 108
+// floats 42 % of the LDS cycles were conflicts); swz keeps those sets and halves the conflicts of the transposing writes.
+__device__ __forceinline__ int swz(int c) { return (c >> 2 & 1) * 12; }
+
+// entry K of the 16-lane windows: its operand row (off: byte offset in LDS, its swizzle in the unit bits; lane16: this
+// lane's 16 l) and its product
+template <int K, int NB>
+__device__ __forceinline__ void entry_load(const char* lds, int off, int lane16, f32x4 (&x)[NB]) {
+  const char* p = lds + (bcast16<K>(off) ^ lane16);
+#pragma unroll
+  for (int h = 0; h < NB; ++h) x[h] = *reinterpret_cast<const f32x4*>(p + 256 * h);
+}
+template <int K, int NB>
+__device__ __forceinline__ void entry_fma(int vb, const f32x4 (&x)[NB], f32x4 (&acc)[NB]) {
+  const float v = __int_as_float(bcast16<K>(vb));
+#pragma unroll
+  for (int h = 0; h < NB; ++h)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc[h][e] += v * x[h][e];
+}
+
+// entries K .. 15 of the windows while fewer than `steps` are done, U operand rows in flight
+template <int K, int U, int NB>
+__device__ __forceinline__ void window(const char* lds, int off, int vb, int lane16, int steps, f32x4 (&acc)[NB]) {
+  if constexpr (K < 16) {
+    if (steps <= K) return;                                  // uniform
+    f32x4 x[U][NB];
+    entry_load<K, NB>(lds, off, lane16, x[0]);
+    if constexpr (U > 1) entry_load<K + 1, NB>(lds, off, lane16, x[1]);
+    if constexpr (U > 2) {
+      entry_load<K + 2, NB>(lds, off, lane16, x[2]);
+      entry_load<K + 3, NB>(lds, off, lane16, x[3]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    entry_fma<K, NB>(vb, x[0], acc);
+    if constexpr (U > 1) entry_fma<K + 1, NB>(vb, x[1], acc);
+    if constexpr (U > 2) {
+      entry_fma<K + 2, NB>(vb, x[2], acc);
+      entry_fma<K + 3, NB>(vb, x[3], acc);
+    }
+    window<K + U, U, NB>(lds, off, vb, lane16, steps, acc);
+  }
+}
+
+// the most entries any of the wave's four rows has in a window, from the lanes that hold one (a prefix of each 16)
+__device__ __forceinline__ int window_steps(unsigned long long m) {
+  const unsigned f = (unsigned)m | (unsigned)(m >> 32);
+  return __popc((f | f >> 16) & 0xffffu);
+}
+
+template <int R, int NB, int U>
 __global__ void __launch_bounds__(1024) spmm_t_kernel(const float* __restrict__ inT, const int* __restrict__ row_ptr,
                                                       const uint16_t* __restrict__ col, const float* __restrict__ val,
                                                       float* __restrict__ outT, const int* __restrict__ omegas,
                                                       int my, int ys, int ncols, int nrows, int rows_out, int compact,
                                                       float alpha, int cspan, int kc, int n_angles, int64_t in_ld,
-                                                      int64_t out_ld, int ys_out) {
-  extern __shared__ float lin[];
-  const int lane = threadIdx.x & 63;
+                                                      int64_t out_ld, int ys_out, int vec_out) {
+  extern __shared__ __align__(16) float lin[];
+  const int lane = threadIdx.x & 63, l16 = lane & 15, lane16 = 16 * l16;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int a = blockIdx.y, s = blockIdx.z;
   const int ra = omegas ? omegas[a] : a;
   const int rr = compact ? a : ra;
-  const int row0 = (blockIdx.x * SPT_WAVES + w) * R;
+  const int rw0 = w * 4 * R + (lane >> 4);                   // row quad i: row rw0 + 4 i of the workgroup's 64 R
+  const int row0 = blockIdx.x * SPT_WAVES * 4 * R + rw0;
   const int c_lo = s * cspan, c_hi = min(ncols, c_lo + cspan);
 
-  // lane l < R: first entry with column >= c_lo and the end of row row0 + l
-  int cur = 0, end = 0;
-  {
-    const int row = row0 + lane;
-    if (lane < R && row < nrows) {
+  // the entries of the workgroup's rows, from one before the first on (so that entry 0 is there whatever the rows hold):
+  // 32-bit offsets to a scalar base
+  const int* wg_ptr = row_ptr + (int64_t)rr * nrows;
+  const int wr0 = blockIdx.x * SPT_WAVES * 4 * R;
+  const int e0 = max(wg_ptr[min(wr0, nrows)] - 1, 0), e1 = wg_ptr[min(wr0 + SPT_WAVES * 4 * R, nrows)];
+  // (no entries so far: the arrays may be empty, and the repeated entry 0 is read from row_ptr instead)
+  const uint16_t* colw = e1 > 0 ? col + e0 : reinterpret_cast<const uint16_t*>(row_ptr);
+  const float* valw = e1 > 0 ? val + e0 : reinterpret_cast<const float*>(row_ptr);
+  // per row: the next entry (the first with column >= c_lo) and the end
+  int cur[R], end[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int row = row0 + 4 * i;
+    cur[i] = end[i] = 0;
+    if (row < nrows) {
       const int64_t rb = (int64_t)rr * nrows + row;
-      int lo = row_ptr[rb], hi = row_ptr[rb + 1];
-      end = hi;
+      int lo = row_ptr[rb] - e0, hi = row_ptr[rb + 1] - e0;
+      end[i] = hi;
       if (c_lo > 0) {
         while (lo < hi) {
           const int mid = (lo + hi) >> 1;
-          if ((int)col[mid] < c_lo) lo = mid + 1;
+          if ((int)colw[mid] < c_lo) lo = mid + 1;
           else hi = mid;
         }
       }
-      cur = lo;
+      cur[i] = lo;
     }
   }
-  // per row: window start we (entry index of lane 0), consumed count wo, end ee; window columns cb and values vw
-  // per lane (one coalesced vector load each; an entry's column and value are then read with v_readlane)
-  int we[R], wo[R], ee[R], cb[R];
-  float vw[R];
-  float acc[R][YW];
+  f32x4 acc[R][NB];
 #pragma unroll
-  for (int i = 0; i < R; ++i) {
-    we[i] = __builtin_amdgcn_readlane(cur, i);
-    ee[i] = __builtin_amdgcn_readlane(end, i);
-    wo[i] = 0;
-    const int idx = we[i] + lane;
-    cb[i] = idx < ee[i] ? (int)col[idx] : 0x7fffffff;
-    vw[i] = idx < ee[i] ? val[idx] : 0.0f;
+  for (int i = 0; i < R; ++i)
 #pragma unroll
-    for (int h = 0; h < YW; ++h) acc[i][h] = 0.f;
-  }
+    for (int h = 0; h < NB; ++h) acc[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const float* lbase = lin + lane;
-  // in_ld > 0: the operand untransposed, (my, in_ld) per angle, transposed while it is staged (ys odd: the
-  // transposing LDS writes, a row of ys floats apart, hit distinct banks); in_ld == 0: transposed, (ncols, ys)
+  // window entry `cu + l16` of a row ending at en (past the end: a repeated entry, not counted)
+  auto fetch = [&](int cu, int en, int& c, float& v) {
+    const unsigned e = (unsigned)max(min(cu + l16, en - 1), 0);
+    c = (int)colw[e];
+    v = valw[e];
+  };
+  int pc0, pc1;
+  float pv0, pv1;
+  fetch(cur[0], end[0], pc0, pv0);
+  fetch(cur[0] + 16, end[0], pc1, pv1);
+
+  // the zero operand
+  constexpr int ROW = 64 * NB;                               // floats of an operand row in LDS
+  const int zoff = kc * ROW * 4;
+  auto row_off = [&](int c) { return c * (ROW * 4) + (swz(c) << 4); };
+  for (int i = threadIdx.x; i < 64 * NB; i += SPT_WAVES * 64) lin[kc * ROW + i] = 0.f;
+
+  // in_ld > 0: the operand untransposed, (my, in_ld) per angle, transposed while it is staged; in_ld == 0: transposed,
+  // (ncols, ys)
   const float* src = in_ld ? inT + (int64_t)a * my * in_ld : inT + (int64_t)a * ncols * ys;
+  const char* lds = reinterpret_cast<const char*>(lin);
   for (int c0 = c_lo; c0 < c_hi; c0 += kc) {
     const int kn = min(kc, c_hi - c0);
     __syncthreads();
-    constexpr int SU = YW >= 7 ? 4 : 8;                      // staging loads in flight per lane
     if (in_ld) {
-      // an item is 4 rows x 64 columns: wave w copies row quads g = w + 16 m, lane (cq_lo + 8 yq + 32 cq_hi) the
-      // float4 of columns 4 cq .. 4 cq + 3 (cq = cq_lo + 8 cq_hi) of row 4 g + yq. c0, in_ld and the base are
-      // multiples of 4 floats, and the columns up to kn rounded up to 4 lie in the row and in the LDS chunk; with
-      // ys odd the 4 transposing writes of a float4 hit distinct banks over every 32 lanes (4 (cq ys mod 8) + yq).
-      const int yq = (lane >> 3) & 3, cq = (lane & 7) + ((lane >> 5) << 3);
-      const int nj = (kn + 63) / 64, ng = (my + 3) / 4;
-      const int items = (ng - w + SPT_WAVES - 1) / SPT_WAVES * nj;
-      for (int it0 = 0; it0 < items; it0 += SU) {
-        float4 v[SU];
+      // an item is 16 rows x 64 columns: a lane loads 4 rows x 4 columns (16-byte loads, 256 contiguous bytes of a row
+      // for the 16 lanes of its row quad) and writes them transposed (16 bytes each). c0, in_ld and the base are
+      // multiples of 4 floats, and the columns up to kn rounded up to 4 lie in the row and in the LDS chunk
+      constexpr int SU = 2;                                  // items in flight per lane
+      const int kq = (lane & 3) + ((lane >> 4) << 2), yq = (lane >> 2) & 3;
+      const int kn4 = (kn + 3) & ~3, nj = (kn + 63) / 64, items = (my + 15) / 16 * nj;
+      for (int it0 = w; it0 < items; it0 += SPT_WAVES * SU) {
+        f32x4 v[SU][4];
 #pragma unroll
         for (int u = 0; u < SU; ++u) {
-          const int it = it0 + u, m = it / nj, kk = 64 * (it - m * nj) + 4 * cq;
-          const int y = 4 * (w + SPT_WAVES * m) + yq;
-          v[u] = (it < items && y < my && kk < kn)
-                     ? *reinterpret_cast<const float4*>(src + (int64_t)y * in_ld + c0 + kk)
-                     : make_float4(0.f, 0.f, 0.f, 0.f);
+          const int it = it0 + SPT_WAVES * u, m = it / nj;
+          const int kk = min(64 * (it - m * nj) + 4 * kq, kn4 - 4), y = 16 * m + 4 * yq;
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            v[u][e] = *reinterpret_cast<const f32x4*>(src + (int64_t)min(y + e, my - 1) * in_ld + c0 + kk);
         }
 #pragma unroll
         for (int u = 0; u < SU; ++u) {
-          const int it = it0 + u, m = it / nj, kk = 64 * (it - m * nj) + 4 * cq;
-          const int y = 4 * (w + SPT_WAVES * m) + yq;
-          if (it < items && y < my && kk < kn) {
-            float* l = lin + kk * ys + y;
-            l[0] = v[u].x;
-            l[ys] = v[u].y;
-            l[2 * ys] = v[u].z;
-            l[3 * ys] = v[u].w;
+          const int it = it0 + SPT_WAVES * u, m = it / nj;
+          const int kk = 64 * (it - m * nj) + 4 * kq, y = 16 * m + 4 * yq;
+          if (kk < kn && y < my) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              *reinterpret_cast<f32x4*>(lin + (kk + e) * ROW + (y ^ swz(kk) * 4)) =
+                  f32x4{v[u][0][e], v[u][1][e], v[u][2][e], v[u][3][e]};
           }
         }
       }
     } else {
-      const float4* g = reinterpret_cast<const float4*>(src + (int64_t)c0 * ys);
-      float4* l4 = reinterpret_cast<float4*>(lin);
-      const int n4 = kn * ys / 4;
+      constexpr int SU = 8;                                  // staging loads in flight per lane
+      const float* g = src + (int64_t)c0 * ys;
+      const int n4 = kn * (ROW / 4);
       for (int i0 = threadIdx.x; i0 < n4; i0 += SPT_WAVES * 64 * SU) {
-        float4 v[SU];
+        f32x4 v[SU];
 #pragma unroll
         for (int u = 0; u < SU; ++u) {
-          const int i = i0 + SPT_WAVES * 64 * u;
-          v[u] = i < n4 ? g[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+          const int i = min(i0 + SPT_WAVES * 64 * u, n4 - 1), c = i / (ROW / 4), y = 4 * (i % (ROW / 4));
+          v[u] = *reinterpret_cast<const f32x4*>(g + (int64_t)c * ys + min(y, ys - 4));
         }
 #pragma unroll
         for (int u = 0; u < SU; ++u) {
-          const int i = i0 + SPT_WAVES * 64 * u;
-          if (i < n4) l4[i] = v[u];
+          const int i = i0 + SPT_WAVES * 64 * u, c = i / (ROW / 4), y = 4 * (i % (ROW / 4));
+          if (i < n4) *reinterpret_cast<f32x4*>(lin + c * ROW + (y ^ swz(c) * 4)) = v[u];
         }
       }
     }
@@ -135,54 +214,52 @@ __global__ void __launch_bounds__(1024) spmm_t_kernel(const float* __restrict__ 
     const int c1 = c0 + kn;
 #pragma unroll
     for (int i = 0; i < R; ++i) {
-      while (true) {
-        const int cnt = __popcll(__ballot(cb[i] < c1));     // entries of the window below c1 (a prefix)
-        const int off = (cb[i] - c0) * ys;                   // operand row offset of each window entry
-        const int vbits = __float_as_int(vw[i]);
-        int t = wo[i];
-        for (; t + U <= cnt; t += U) {                        // U operand rows in flight, summed in entry order
-          float x[U][YW], v[U];
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const float* lp = lbase + __builtin_amdgcn_readlane(off, t + u);
-            v[u] = __int_as_float(__builtin_amdgcn_readlane(vbits, t + u));
-#pragma unroll
-            for (int h = 0; h < YW; ++h) x[u][h] = lp[64 * h];
-          }
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int h = 0; h < YW; ++h) acc[i][h] += v[u] * x[u][h];
+      bool in0 = cur[i] + l16 < end[i] && pc0 < c1, in1 = cur[i] + 16 + l16 < end[i] && pc1 < c1;
+      const int off0 = in0 ? row_off(pc0 - c0) : zoff, off1 = in1 ? row_off(pc1 - c0) : zoff;
+      const int vb0 = in0 ? __float_as_int(pv0) : 0, vb1 = in1 ? __float_as_int(pv1) : 0;
+      const unsigned long long m0 = __ballot(in0), m1 = __ballot(in1);
+      const int shift = lane & 48;
+      const int n = __popc((unsigned)(m0 >> shift) & 0xffffu) + __popc((unsigned)(m1 >> shift) & 0xffffu);
+      cur[i] += n;
+      // the next visit's windows (the last row quad: the first one's in the next chunk)
+      fetch(cur[i + 1 < R ? i + 1 : 0], end[i + 1 < R ? i + 1 : 0], pc0, pv0);
+      fetch(cur[i + 1 < R ? i + 1 : 0] + 16, end[i + 1 < R ? i + 1 : 0], pc1, pv1);
+      __builtin_amdgcn_sched_barrier(0);
+      window<0, U, NB>(lds, off0, vb0, lane16, window_steps(m0), acc[i]);
+      if (m1) window<0, U, NB>(lds, off1, vb1, lane16, window_steps(m1), acc[i]);
+      bool more = __any(n == 32);
+      while (more) {                                         // a row with more than 32 entries in the chunk
+        int c;
+        float v;
+        fetch(cur[i], end[i], c, v);
+        const bool in = cur[i] + l16 < end[i] && c < c1;
+        const unsigned long long m = __ballot(in);
+        window<0, U, NB>(lds, in ? row_off(c - c0) : zoff, in ? __float_as_int(v) : 0, lane16, window_steps(m),
+                         acc[i]);
+        const int nn = __popc((unsigned)(m >> shift) & 0xffffu);
+        cur[i] += nn;
+        more = __any(nn == 16);
+        if (R == 1) {                                        // the next visit is this row's
+          fetch(cur[0], end[0], pc0, pv0);
+          fetch(cur[0] + 16, end[0], pc1, pv1);
         }
-        for (; t < cnt; ++t) {
-          const float* lp = lbase + __builtin_amdgcn_readlane(off, t);
-          const float vt = __int_as_float(__builtin_amdgcn_readlane(vbits, t));
-#pragma unroll
-          for (int h = 0; h < YW; ++h) acc[i][h] += vt * lp[64 * h];
-        }
-        wo[i] = cnt;
-        if (cnt < 64 || we[i] + 64 >= ee[i]) break;
-        we[i] += 64;                                       // window used up: the next 64 entries
-        wo[i] = 0;
-        const int idx = we[i] + lane;
-        cb[i] = idx < ee[i] ? (int)col[idx] : 0x7fffffff;
-        vw[i] = idx < ee[i] ? val[idx] : 0.0f;
       }
     }
   }
 
   if (out_ld) {
-    // out (n_angles, my, out_ld): per group of 64 y, the workgroup's RB = 16 R rows go through LDS as (y, row) with
+    // out (n_angles, my, out_ld): per group of 64 y, the workgroup's RB = 64 R rows go through LDS as (y, row) with
     // the odd row stride RB + 1 (64 (RB + 1) floats), then out one y row of RB consecutive floats at a time
-    constexpr int RB = SPT_WAVES * R, RW = RB + 1;
+    constexpr int RB = SPT_WAVES * 4 * R, RW = RB + 1;
     const int r = threadIdx.x % RB, row = blockIdx.x * RB + r;
     float* dst = outT + (int64_t)a * my * out_ld;
 #pragma unroll
-    for (int h = 0; h < YW; ++h) {
+    for (int h = 0; h < NB; ++h) {
       __syncthreads();
 #pragma unroll
-      for (int i = 0; i < R; ++i) lin[lane * RW + w * R + i] = alpha * acc[i][h];
+      for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) lin[(4 * l16 + e) * RW + rw0 + 4 * i] = alpha * acc[i][h][e];
       __syncthreads();
       if (row < rows_out)
         for (int yl = threadIdx.x / RB; yl < 64 && 64 * h + yl < my; yl += SPT_WAVES * 64 / RB)
@@ -193,12 +270,20 @@ __global__ void __launch_bounds__(1024) spmm_t_kernel(const float* __restrict__ 
   float* dst = outT + ((int64_t)s * n_angles + a) * rows_out * ys_out;
 #pragma unroll
   for (int i = 0; i < R; ++i) {
-    const int row = row0 + i;
+    const int row = row0 + 4 * i;
     if (row < rows_out) {
 #pragma unroll
-      for (int h = 0; h < YW; ++h) {
-        const int y = 64 * h + lane;
-        if (y < my) dst[(int64_t)row * ys_out + y] = alpha * acc[i][h];
+      for (int h = 0; h < NB; ++h) {
+        const int y = 64 * h + 4 * l16;
+        float* d = dst + (int64_t)row * ys_out + y;
+        const f32x4 v = alpha * acc[i][h];
+        if (vec_out && y + 3 < my) {
+          *reinterpret_cast<f32x4*>(d) = v;
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (y + e < my) d[e] = v[e];
+        }
       }
     }
   }
@@ -239,48 +324,70 @@ __global__ void __launch_bounds__(256) transpose_sum_kernel(const float* __restr
   }
 }
 
-template <int R, int YW>
+template <int R, int NB>
 void launch_spmm_t(dim3 grid, size_t lds, hipStream_t st, const float* inT, const int* row_ptr, const uint16_t* col,
                    const float* val, float* outT, const int* omegas, int my, int ys, int ncols, int nrows,
                    int rows_out, int compact, float alpha, int cspan, int kc, int n_angles, int64_t in_ld,
                    int64_t out_ld, int ys_out) {
-  hipLaunchKernelGGL((spmm_t_kernel<R, YW, (YW <= 4 ? 8 : 4)>), grid, dim3(SPT_WAVES * 64), lds, st, inT, row_ptr,
-                     col, val, outT, omegas, my, ys, ncols, nrows, rows_out, compact, alpha, cspan, kc, n_angles,
-                     in_ld, out_ld, ys_out);
+  const int vec_out = ys_out % 4 == 0 && (uintptr_t)outT % 16 == 0;
+  hipLaunchKernelGGL((spmm_t_kernel<R, NB, (NB <= 2 ? 4 : NB <= 4 ? 2 : 1)>), grid, dim3(SPT_WAVES * 64), lds, st,
+                     inT, row_ptr, col, val, outT, omegas, my, ys, ncols, nrows, rows_out, compact, alpha, cspan, kc,
+                     n_angles, in_ld, out_ld, ys_out, vec_out);
 }
 
-// ys: the LDS row stride (the transposed input's row stride when in_ld == 0); ys_out: the transposed output's
+// row quads per wave: 4 (256 rows a workgroup), 2 where the accumulators of more than 128 detector positions leave no
+// registers for more (128 VGPRs with 16 waves on a CU)
+int row_quads(int my) { return my <= 128 ? 4 : 2; }
+
+// ... and fewer where that leaves workgroups for less than half of the 256 CUs (a workgroup's LDS fills one): the operand
+// is staged again for each, the rows' serial walks shorten (us, 900 segments x 103 rows, 256 / fewer rows: adjoint, 333
+// orientations x 50 angles 92 / 62, 1500 x 18 63 / 45; forward in one range, 1500 x 18 92 / 64; with 256 workgroups as
+// the line 54 instead of 45, 73 instead of 64)
+int row_quads(int my, int64_t rows_out, int64_t others) {
+  int R = row_quads(my);
+  while (R > 1 && (rows_out + 64 * R - 1) / (64 * R) * others < 128) R /= 2;
+  return R;
+}
+
+// ys: the transposed input's row stride (in_ld == 0); ys_out: the transposed output's
 int spmm_t_impl(const float* in, int64_t in_ld, const int32_t* row_ptr, const uint16_t* col, const float* val,
                 float* out, int64_t out_ld, int32_t ys_out, const int32_t* omegas, int32_t n_angles, int32_t my,
                 int32_t ys, int32_t ncols, int32_t nrows, int32_t rows_out, int32_t compact, float alpha,
                 int32_t nsplit, int32_t kc, hipStream_t st) {
-  const int kc_max = (SPT_LDS_FLOATS - 64) / ys;
+  const int nb = (my + 63) / 64;
+  const int row = 64 * nb;           // floats of an operand row in LDS
+  const int kc_max = SPT_LDS_FLOATS / row - 1;
   if (kc <= 0 || kc > kc_max) kc = kc_max;
   int cspan = (ncols + nsplit - 1) / nsplit;
-  if (in_ld) {                       // float4 staging of the untransposed operand: chunks start at multiples of 4
-    kc &= ~3;
+  if (in_ld) {                       // 16-byte staging of the untransposed operand: chunks start at multiples of 4
+    kc = std::max(kc & ~3, 4);
     cspan = (cspan + 3) & ~3;
   }
+  kc = std::min(kc, in_ld ? cspan : std::min(cspan, ncols));
   if (n_angles == 0 || rows_out == 0) return DFM_OK;
-  const int yw = (my + 63) / 64;
-  const int R = my <= 128 ? 16 : 8;   // 16 rows of 3 y groups would spill with the value windows
-  const dim3 grid((unsigned)((rows_out + SPT_WAVES * R - 1) / (SPT_WAVES * R)), (unsigned)n_angles,
+  const int R = row_quads(my, rows_out, (int64_t)n_angles * nsplit);
+  const dim3 grid((unsigned)((rows_out + SPT_WAVES * 4 * R - 1) / (SPT_WAVES * 4 * R)), (unsigned)n_angles,
                   (unsigned)nsplit);
-  size_t lds = ((size_t)kc * ys + 64) * sizeof(float);
-  if (out_ld) lds = std::max(lds, (size_t)64 * (SPT_WAVES * R + 1) * sizeof(float));
+  size_t lds = (size_t)(kc + 1) * row * sizeof(float);
+  if (out_ld) lds = std::max(lds, (size_t)64 * (SPT_WAVES * 4 * R + 1) * sizeof(float));
 #define DFM_SPT(RR, YY)                                                                                      \
   launch_spmm_t<RR, YY>(grid, lds, st, in, row_ptr, col, val, out, omegas, my, ys, ncols, nrows, rows_out,  \
                         compact, alpha, cspan, kc, n_angles, in_ld, out_ld, ys_out)
-  switch (yw) {
-    case 1: DFM_SPT(16, 1); break;
-    case 2: DFM_SPT(16, 2); break;
-    case 3: DFM_SPT(8, 3); break;
-    case 4: DFM_SPT(8, 4); break;
-    case 5: DFM_SPT(8, 5); break;
-    case 6: DFM_SPT(8, 6); break;
-    case 7: DFM_SPT(8, 7); break;
-    default: DFM_SPT(8, 8); break;
+#define DFM_SPT_R(YY, RMAX)                                   \
+  if (R == RMAX) DFM_SPT(RMAX, YY);                           \
+  else if (R == 2) DFM_SPT(2, YY);                            \
+  else DFM_SPT(1, YY)
+  switch (nb) {
+    case 1: DFM_SPT_R(1, 4); break;
+    case 2: DFM_SPT_R(2, 4); break;
+    case 3: DFM_SPT_R(3, 2); break;
+    case 4: DFM_SPT_R(4, 2); break;
+    case 5: DFM_SPT_R(5, 2); break;
+    case 6: DFM_SPT_R(6, 2); break;
+    case 7: DFM_SPT_R(7, 2); break;
+    default: DFM_SPT_R(8, 2); break;
   }
+#undef DFM_SPT_R
 #undef DFM_SPT
   return DFM_OK;
 }
@@ -291,7 +398,7 @@ extern "C" {
 
 int dfm_spmm_t_rows_per_block(int32_t my) {
   if (my <= 0 || my > 512) return 0;
-  return SPT_WAVES * (my <= 128 ? 16 : 8);
+  return SPT_WAVES * 4 * row_quads(my);
 }
 
 int dfm_spmm_t(const float* inT, const int32_t* row_ptr, const uint16_t* col, const float* val, float* outT,
@@ -328,8 +435,7 @@ int dfm_spmm_t_direct(const float* in, int64_t in_ld, int32_t in_ys, const int32
     dfm::set_error("dfm_spmm_t_direct: the input must be 16-byte aligned, in_ld a multiple of 4");
     return DFM_ERR_ARG;
   }
-  const int ys = in_ld ? (my | 1) : in_ys;     // odd LDS row stride for the transposing staging
-  spmm_t_impl(in, in_ld, row_ptr, col, val, out, out_ld, out_ys, omegas, n_angles, my, ys, ncols, nrows, rows_out,
+  spmm_t_impl(in, in_ld, row_ptr, col, val, out, out_ld, out_ys, omegas, n_angles, my, in_ys, ncols, nrows, rows_out,
               compact, alpha, nsplit, kc, (hipStream_t)stream);
   DFM_LAUNCH_CHECK("dfm_spmm_t_direct");
   return DFM_OK;

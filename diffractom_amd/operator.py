@@ -13,6 +13,7 @@ the whole run.
 from __future__ import annotations
 
 import ctypes
+import functools
 import time
 from typing import Any, Mapping
 
@@ -1052,8 +1053,8 @@ class SinglePhaseForwardOperator:
         and its chain of lines cost what they save or more (72 x 72 x 512 x 18 31 / 26, 64 x 64 x 6016 x 6 68 / 58, 32 x
         32 x 512 x 18 17 / 9). Otherwise the table, in bands for large images."""
         n = max(self.Nx, self.Ny)
-        if tab is not None and tab["pairs_ok"] and n <= 256 and \
-                (n > 80 or self.Nx * self.Ny * n_angles * kn >= 150_000_000):
+        if (n > 80 or self.Nx * self.Ny * n_angles * kn >= 150_000_000) and tab is not None and n <= 256 and \
+                tab["pairs_ok"]:
             return "lines"
         return "band" if self.radon_bands >= 4 else "table"
 
@@ -1270,8 +1271,8 @@ class SinglePhaseForwardOperator:
             data = torch.rand(self.data_shape, generator=g, device=dev)
             times = {}
             cands = {}
-            if _lib.load().dfm_spmm_t_rows_per_block(self.My) > 0:
-                cands.update({f"t:split:{k}": dict(fwd="t", tsplit=k) for k in (16, 8, 4, 32)})
+            if self._t_rows > 0:
+                cands.update({f"t:split:{k}": dict(fwd="t", tsplit=k) for k in (1, 2, 4, 8, 16)})
             cands.update({f"rows:ksplit:{k},kc:{c}": dict(fwd="rows", ksplit=k, kc=c) for k in (16, 4)
                           for c in (256, 768)})
             for name, v in cands.items():
@@ -1281,7 +1282,7 @@ class SinglePhaseForwardOperator:
             self.csr_variant.update(cands[best])
             out["pf_forward"] = (best, times)
             times = {}
-            for name in (("t", "rows") if _lib.load().dfm_spmm_t_rows_per_block(self.My) > 0 else ("rows",)):
+            for name in (("t", "rows") if self._t_rows > 0 else ("rows",)):
                 self.csr_variant["adj"] = name
                 times[name] = timeit(lambda: self._pf_adjoint(0, data, sc["sino"], subset))
             best = _pick(times)
@@ -1447,8 +1448,13 @@ class SinglePhaseForwardOperator:
         """"t" (wavefront-segmented kernel on transposed operands) or "rows" (a thread per CSR row)."""
         v = self.csr_variant.get(direction, "auto")
         if v == "auto":
-            return "t" if _lib.load().dfm_spmm_t_rows_per_block(self.My) > 0 else "rows"
+            return "t" if self._t_rows > 0 else "rows"
         return v
+
+    @functools.cached_property
+    def _t_rows(self):
+        """The most CSR rows per workgroup of the transposed products (0: more detector rows than they take)."""
+        return int(_lib.load().dfm_spmm_t_rows_per_block(self.My))
 
     @property
     def _ys(self):
@@ -1468,13 +1474,18 @@ class SinglePhaseForwardOperator:
         return [p[o:o + int(z)] for o, z in zip(offs, sizes)]
 
     def _tsplit(self, n_ang, kb):
-        """Orientation split of the transposed forward: enough workgroups for 4 per CU on 256 CUs."""
+        """Orientation split of the transposed forward: 64 workgroups of the most rows (the kernel takes fewer rows in
+        each, down to a quarter, where they are fewer than 128; a workgroup's LDS fills a CU), in ranges of 256
+        orientations or more, for every split writes and adds up a partial result (us for a split of 1 / 2 / 4, 900
+        segments x 103 rows: 9899 orientations x 180 angles 1630 / 1724 / 1905, 1500 x 18 64 / 66 / 72, 543 x 23 25 / 27
+        / 39). Below 1024 workgroups, ranges of at most 5120 orientations, which bounds the FP32 chains: at 9899 x 180 one
+        range is 5 % faster and twice as far from 64 bits (3.8e-7 against 2.0e-7)."""
         v = self.csr_variant.get("tsplit", "auto")
         if v != "auto":
             return int(max(1, min(int(v), max(kb, 1))))
-        rpb = _lib.load().dfm_spmm_t_rows_per_block(self.My)
-        wgs = -(-self.N_seg // rpb) * n_ang
-        return int(max(1, min(64, -(-1024 // wgs), max(kb // 128, 1))))
+        wgs = -(-self.N_seg // self._t_rows) * n_ang
+        ns = max(min(-(-64 // wgs), max(kb // 256, 1)), min(-(-1024 // wgs), -(-kb // 5120)))
+        return int(max(1, min(64, ns)))
 
     def _spmm_t_forward(self, b, sb, om, n_ang, sino, data, accumulate):
         """sino (n_ang, my, kstride) -> split partials (ns, n_ang, cp, ys) -> data rows; the sinogram is transposed

@@ -173,8 +173,8 @@ int dfm_spmm_forward_split(const float* sino, const int32_t* row_ptr, const uint
                            float* data, const int32_t* omegas, int32_t n_angles, int32_t my, int32_t cp,
                            int32_t kstride, int32_t kb, int32_t compact, int32_t accumulate, float* part,
                            int32_t ksplit, int32_t kc, dfm_stream_t stream);
-/* The same products on transposed operands (wavefront-segmented SpMM: a wave per R CSR rows, lanes over y, column
- * chunks of the operand staged in LDS), for either CSR form:
+/* The same products on transposed operands (wavefront-segmented SpMM: 16 lanes per CSR row, 4 y of every 64 each,
+ * column chunks of the operand staged in LDS), for either CSR form:
  *   outT[s, a, row, y] = alpha sum_{e in row (rr, row), col(e) in split s} val[e] inT[a, col(e), y]
  * with rr = a if compact else omegas[a]; inT (n_angles, ncols, ys), outT (nsplit, n_angles, rows_out, ys), ys >= my a
  * multiple of 4, inT 16-byte aligned; split s covers columns [s cspan, (s + 1) cspan), cspan = ceil(ncols / nsplit);
@@ -193,7 +193,7 @@ int dfm_spmm_t_direct(const float* in, int64_t in_ld, int32_t in_ys, const int32
                       const float* val, float* out, int64_t out_ld, int32_t out_ys, const int32_t* omegas,
                       int32_t n_angles, int32_t my, int32_t ncols, int32_t nrows, int32_t rows_out, int32_t compact,
                       float alpha, int32_t nsplit, int32_t kc, dfm_stream_t stream);
-/* CSR rows per workgroup of dfm_spmm_t for a given my (0: my unsupported). */
+/* The most CSR rows per workgroup of dfm_spmm_t for a given my (0: my unsupported). */
 int dfm_spmm_t_rows_per_block(int32_t my);
 /* out[ao, c, r] (+)= sum_{s < nsplit} in[s split_stride + ai in_mat + r in_ld + c] for a = 0 .. n_mat-1, with
  * ai = omegas[a] if omegas and omega_out == 0, ao = omegas[a] if omegas and omega_out == 1, else a. */
