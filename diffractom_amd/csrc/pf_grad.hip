@@ -17,6 +17,13 @@
 // an My-long dot (float64) and the entry's derivative terms (float64, as pf_entry), accumulated per orientation in
 // LDS (float64 atomics) and written per (angle, orientation); the per-workgroup sums of the global parameters go to
 // a partial array. dfm_pf_grad_reduce sums both over angles / workgroups in a fixed order.
+//
+// What bounds it: load latency (waves wait 79 % of their cycles, VALU 27 -> 39 % busy). So an axis is loaded while the
+// one before is evaluated, the directions' derivatives are read once per node and multiply the axes' summed n dg/dd
+// (instead of 12 loads per contributing axis), the dot's and the staging's loads go ahead, the global parameters' sums
+// stay in registers until the end (they were 64-way conflicts on one LDS word), and 128 VGPRs keep four workgroups on a
+// CU (142 without the limit: 3; 1.46 -> 0.96 ms with the sums). 60 angles x 1,000 orientations x 67 rows, five rings:
+// 1.76 -> 0.96 ms.
 #include "pf_cand.h"
 
 namespace {
@@ -42,7 +49,7 @@ struct GradArgs {
   int n_ang, n_kb, n_jb, Se, My, CP, sks, nqk, hess;
 };
 
-__global__ void __launch_bounds__(GR_THREADS) pf_grad_kernel(GradArgs g) {
+__global__ void __launch_bounds__(GR_THREADS, 4) pf_grad_kernel(GradArgs g) {
   extern __shared__ unsigned gr_lds[];
   const dfm::CandGeo& cg = g.cg;
   const int W = 32 * g.n_jb;
@@ -100,15 +107,17 @@ __global__ void __launch_bounds__(GR_THREADS) pf_grad_kernel(GradArgs g) {
 
   const int CPn = g.CP, P = cg.P, A = cg.A, S = cg.S, Se = g.Se;
   const double inv_nodes = 1.0 / (double)(S * Se);
+  double sum_g[3] = {0.0, 0.0, 0.0};                           // eta, tilt 0, tilt 1: this thread's candidates
   for (int jb = 0; jb < g.n_jb; ++jb) {
     const int c_lo = pre[jb * 32], c_hi = pre[jb * 32 + 32];
     if (c_lo == c_hi) continue;                                // uniform
-    for (int i = tid; i < g.My * 32; i += GR_THREADS) {
-      const int y = i >> 5, jl = i & 31, j = jb * 32 + jl;
-      const int64_t o = ((int64_t)r * g.My + y) * CPn + j;
-      rb[i] = j < CPn ? g.r[o] : 0.f;
-      if (g.hess) cb[i] = j < CPn ? g.curv[o] : 0.f;
-    }
+    // (segments beyond the last repeat it; they are no candidates)
+    const int64_t o = (int64_t)r * g.My * CPn + min(jb * 32 + (tid & 31), CPn - 1);
+#pragma unroll 8
+    for (int i = tid; i < g.My * 32; i += GR_THREADS) rb[i] = g.r[o + (int64_t)(i >> 5) * CPn];
+    if (g.hess)
+#pragma unroll 8
+      for (int i = tid; i < g.My * 32; i += GR_THREADS) cb[i] = g.curv[o + (int64_t)(i >> 5) * CPn];
     __syncthreads();
     for (int ci = c_lo + tid; ci < c_hi; ci += GR_THREADS) {
       // the candidate's word (the last of the block's 32 with pre[w] <= ci) and bit (the rank-th set bit)
@@ -124,10 +133,16 @@ __global__ void __launch_bounds__(GR_THREADS) pf_grad_kernel(GradArgs g) {
       const int c = j / P, p = j - c * P;
       const int kg = cg.k0 + kbi * 32 + kl;
       double G = 0.0, C2 = 0.0;
-      for (int y = 0; y < g.My; ++y) {
-        const double sv = sb[y * 32 + kl];
-        G += sv * (double)rb[y * 32 + jl];
-        if (g.hess) C2 += sv * sv * (double)cb[y * 32 + jl];
+      if (g.hess) {                                            // (uniform, outside: the loops' LDS reads go ahead)
+#pragma unroll 4
+        for (int y = 0; y < g.My; ++y) {
+          const double sv = sb[y * 32 + kl];
+          G += sv * (double)rb[y * 32 + jl];
+          C2 += sv * sv * (double)cb[y * 32 + jl];
+        }
+      } else {
+#pragma unroll 8
+        for (int y = 0; y < g.My; ++y) G += (double)sb[y * 32 + kl] * (double)rb[y * 32 + jl];
       }
       const double is2 = cg.inv_sigma2[kg], nk = g.normf[kg];
       const double sig_fac1 = -2.0 * sqrt(is2), sig_fac3 = -2.0 * is2 * sqrt(is2);   // -2 / sigma, -2 / sigma^3
@@ -139,26 +154,38 @@ __global__ void __launch_bounds__(GR_THREADS) pf_grad_kernel(GradArgs g) {
           const int64_t vo = (((((int64_t)r * S + s) * cg.C + c) * Se + se) * P + p) * 3;
           const double vx = g.coords[vo], vy = g.coords[vo + 1], vz = g.coords[vo + 2];
           const double wn = (g.qw ? (double)g.qw[s * Se + se] : inv_nodes) * nk;
+          // the node's sum of m dg/dd n over the axes: the directions' derivatives multiply it once
+          double tx = 0.0, ty = 0.0, tz = 0.0;
+          const int af = min(a0, A - 1);
+          double nx = pk[af * 3], ny = pk[af * 3 + 1], nz = pk[af * 3 + 2], cnt = (double)g.axis_count[af];
           for (int ax = a0; ax < a1; ++ax) {
-            const double nx = pk[ax * 3], ny = pk[ax * 3 + 1], nz = pk[ax * 3 + 2];
-            const double d = nx * vx + ny * vy + nz * vz, ad = fabs(d);
+            const double ux = nx, uy = ny, uz = nz, mult = cnt;
+            const int nxt = min(ax + 1, a1 - 1);               // the next axis is loaded while this one is evaluated
+            nx = pk[nxt * 3];
+            ny = pk[nxt * 3 + 1];
+            nz = pk[nxt * 3 + 2];
+            cnt = (double)g.axis_count[nxt];
+            const double d = ux * vx + uy * vy + uz * vz, ad = fabs(d);
             const double x1 = (1.0 - ad) * is2, x2 = (1.0 + ad) * is2;
             const double e1 = x1 < cg.cut ? exp(-x1) : 0.0, e2 = x2 < cg.cut ? exp(-x2) : 0.0;
             if (e1 == 0.0 && e2 == 0.0) continue;
-            const double m = (double)g.axis_count[ax] * wn;
+            const double m = mult * wn;
             const double dgd = (d < 0.0 ? -is2 : is2) * (e1 - e2) * m;
             const double gv = (e1 + e2) * m, dgs = (-(1.0 - ad) * e1 - (1.0 + ad) * e2) * m;
-            J0 += dgd * (ny * vz - nz * vy);                  // n x v
-            J1 += dgd * (nz * vx - nx * vz);
-            J2 += dgd * (nx * vy - ny * vx);
+            tx += dgd * ux;
+            ty += dgd * uy;
+            tz += dgd * uz;
             J3 += sig_fac1 * gv + sig_fac3 * dgs;
-            if (g.dv_eta) ge += dgd * (nx * g.dv_eta[vo] + ny * g.dv_eta[vo + 1] + nz * g.dv_eta[vo + 2]);
-            if (g.dv_t0) {
-              gt0 += dgd * (nx * g.dv_t0[vo] + ny * g.dv_t0[vo + 1] + nz * g.dv_t0[vo + 2]);
-              gt1 += dgd * (nx * g.dv_t1[vo] + ny * g.dv_t1[vo + 1] + nz * g.dv_t1[vo + 2]);
-            }
-            if (g.dv_tth) gtt += dgd * (nx * g.dv_tth[vo] + ny * g.dv_tth[vo + 1] + nz * g.dv_tth[vo + 2]);
           }
+          J0 += ty * vz - tz * vy;                             // n x v
+          J1 += tz * vx - tx * vz;
+          J2 += tx * vy - ty * vx;
+          if (g.dv_eta) ge += tx * g.dv_eta[vo] + ty * g.dv_eta[vo + 1] + tz * g.dv_eta[vo + 2];
+          if (g.dv_t0) {
+            gt0 += tx * g.dv_t0[vo] + ty * g.dv_t0[vo + 1] + tz * g.dv_t0[vo + 2];
+            gt1 += tx * g.dv_t1[vo] + ty * g.dv_t1[vo + 1] + tz * g.dv_t1[vo + 2];
+          }
+          if (g.dv_tth) gtt += tx * g.dv_tth[vo] + ty * g.dv_tth[vo + 1] + tz * g.dv_tth[vo + 2];
         }
       }
       double* ak = acc_k + kl * g.nqk;
@@ -174,15 +201,19 @@ __global__ void __launch_bounds__(GR_THREADS) pf_grad_kernel(GradArgs g) {
 #pragma unroll
           for (int v = u; v < 4; ++v) atomicAdd(ak + q++, C2 * Jv[u] * Jv[v]);
       }
-      if (g.dv_eta) atomicAdd(acc_g + 0, G * ge);
-      if (g.dv_t0) {
-        atomicAdd(acc_g + 1, G * gt0);
-        atomicAdd(acc_g + 2, G * gt1);
-      }
+      sum_g[0] += G * ge;                                      // (0 where the group is not asked for)
+      sum_g[1] += G * gt0;
+      sum_g[2] += G * gt1;
       if (g.dv_tth) atomicAdd(acc_g + 3 + p, G * gtt);
     }
     __syncthreads();                                           // rb / cb are staged again for the next block
   }
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    for (int off = 32; off > 0; off >>= 1) sum_g[q] += __shfl_down(sum_g[q], off, 64);
+    if (lane == 0) atomicAdd(acc_g + q, sum_g[q]);
+  }
+  __syncthreads();
   for (int i = tid; i < 32 * g.nqk; i += GR_THREADS) {
     const int kl = i / g.nqk, kloc = kbi * 32 + kl;
     if (kloc < cg.kb) g.part_k[((int64_t)a * cg.kb + kloc) * g.nqk + (i - kl * g.nqk)] = acc_k[i];
