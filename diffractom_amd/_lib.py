@@ -141,7 +141,7 @@ def exported_symbols():
 
 def call(name, *args):
     """Call an entry point; a non-zero status raises the matching exception with the library's message."""
-    lib = load()
+    lib = _lib or load()
     st = getattr(lib, name)(*args)
     if st != 0:
         msg = lib.dfm_last_error().decode(errors="replace")
@@ -159,11 +159,13 @@ MAX_PARTIALS = 2048   # DFM_MAX_PARTIALS of the header: partial sums a reduction
 
 
 def ptr(t):
-    """Device pointer of a torch tensor (None -> NULL)."""
-    return None if t is None else c_void_p(t.data_ptr())
+    """Device pointer of a torch tensor (None -> NULL), as the number the entry points' void * arguments take."""
+    return None if t is None else t.data_ptr()
 
 
 def stream_handle(stream=None):
     import torch
-    s = torch.cuda.current_stream() if stream is None else stream
-    return c_void_p(s.cuda_stream)
+    # (the raw handle: a Stream object a call, several calls a pass, was a tenth of the host time of the smallest
+    # products, which are bound by it: 16 x 16 pixels, 12 orientations, 30 angles, four launches)
+    s = torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()) if stream is None else stream.cuda_stream
+    return c_void_p(s)

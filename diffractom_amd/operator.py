@@ -1483,6 +1483,8 @@ class SinglePhaseForwardOperator:
         v = self.csr_variant.get("tsplit", "auto")
         if v != "auto":
             return int(max(1, min(int(v), max(kb, 1))))
+        if kb < 512:
+            return 1
         wgs = -(-self.N_seg // self._t_rows) * n_ang
         ns = max(min(-(-64 // wgs), max(kb // 256, 1)), min(-(-1024 // wgs), -(-kb // 5120)))
         return int(max(1, min(64, ns)))
