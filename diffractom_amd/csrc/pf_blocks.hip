@@ -604,6 +604,8 @@ int dfm_pfblk_forward(const float* sino, int32_t sks, int32_t kb, const int32_t*
                 "dfm_pfblk_forward: mode %d (0 bf16, 1 bf16 residual, 2 fp16 with ring scales)", mode);
   DFM_CHECK_ARG(n_ang > 0 && my > 0 && cp > 0 && kb > 0 && sks >= kb && (sks & 3) == 0,
                 "dfm_pfblk_forward: bad sizes (n_ang %d, My %d, CP %d, Kb %d, stride %d)", n_ang, my, cp, kb, sks);
+  DFM_CHECK_ARG((int64_t)(my < 32 ? my : 32) * sks < (int64_t)1 << 30,
+                "dfm_pfblk_forward: sinogram rows of %d floats (32 of them pass 4 GiB)", sks);
   BlkArgs p{};
   p.blk_local = local;
   p.n_kb = (kb + 31) / 32;
