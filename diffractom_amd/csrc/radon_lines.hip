@@ -36,10 +36,16 @@ struct LineGeo {
 
 // 16 bytes a lane from global memory to dst + 16 lane in LDS; lanes off by exec write nothing. In assembly because the
 // compiler waits for every such load before the next LDS read, whatever its address. It has no register output; the
-// caller waits (vmcnt) before the barrier that hands the data over.
+// caller waits (vmcnt) before the barrier that hands the data over. The load takes its LDS address from M0, whose scalar
+// write needs one wait state before it: without the s_nop the load may still see the M0 of the load before, and the
+// compiler adds none inside assembly. M0 is named as written (a reserved register: hence the warning that is off).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void lds_load16(const float4* p, unsigned dst) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(p), "s"(dst) : "memory");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(p), "s"(dst)
+               : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 template <bool DUP>
 __global__ void __launch_bounds__(TH, 4) radon_forward_lines_kernel(
