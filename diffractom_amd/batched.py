@@ -111,7 +111,7 @@ class BatchedSPDHGPoisson:
         # eagerly once and capturing it the second time (the launches of a step: dual update, grouped PF adjoint,
         # backprojection, forward projection, grouped PF forward; no host work, no allocation, no memset)
         self.graphs = bool(graphs)
-        self._graph_cache, self._graph_seen = {}, set()
+        self._graph_cache, self._graph_seen, self._graph_gen = {}, set(), None
 
     # ---------------------------------------------------------------- order (spdhg_poisson.py:363-370)
     _epoch_order = SPDHGPoisson._epoch_order
@@ -319,6 +319,7 @@ class BatchedSPDHGPoisson:
         if not self.graphs or full or self.ops[0].queue is not None:
             self.step(nb, full_forward=full)
             return
+        self._check_graphs()
         key = (blk, nb)
         g = self._graph_cache.get(key)
         if g is None and key in self._graph_seen:
@@ -329,16 +330,30 @@ class BatchedSPDHGPoisson:
         else:
             g.replay()
 
+    def _check_graphs(self):
+        """Forget the captured steps when a workspace of the operator that launches them was replaced: they write to
+        the old one."""
+        gen = getattr(self.ops[0], "scratch_generation", 0)
+        if gen != self._graph_gen:
+            self._graph_cache.clear()
+            self._graph_seen.clear()
+            self._graph_gen = gen
+
     def _capture(self, blk, nb):
+        """The captured step, or None (and no captured steps) when a workspace was allocated while capturing."""
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g):
             self.step(nb, block=blk)
+        if getattr(self.ops[0], "scratch_generation", 0) != self._graph_gen:
+            self._check_graphs()
+            return None
         self._graph_cache[(blk, nb)] = g
         return g
 
     def capture_all(self):
         """Capture the step of every ordered pair of distinct subsets (graphs on; after start()): the descriptors
-        and tables of every subset are made first, eagerly, so nothing is allocated while capturing. Returns the
+        and tables of every subset are made first, eagerly, so nothing is allocated while capturing; where a workspace
+        grows all the same (the bands of a larger subset), the steps captured before are captured again. Returns the
         number of graphs."""
         if not self.graphs:
             raise ValueError("capture_all needs graphs=True")
@@ -348,10 +363,13 @@ class BatchedSPDHGPoisson:
             self._group(False, m)
             o0._tables(m)
         torch.cuda.synchronize(o0.device)
-        for a in range(self.M):
-            for b in range(self.M):
-                if a != b and (a, b) not in self._graph_cache:
-                    self._capture(a, b)
+        self._check_graphs()
+        todo = True
+        while todo:
+            todo = [(a, b) for a in range(self.M) for b in range(self.M) if a != b and (a, b) not in self._graph_cache]
+            for a, b in todo:
+                if self._capture(a, b) is None:
+                    break
         return len(self._graph_cache)
 
     def advance(self, n_steps):

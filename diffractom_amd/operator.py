@@ -1074,15 +1074,16 @@ class SinglePhaseForwardOperator:
         return nsplit, int(n <= 128)
 
     def _lines_part(self, tab, n_angles, kn):
-        """Floats of the line sweep's partial sinograms, the most any subset needs (so that the workspace does not
-        grow between the subsets of a run, whose steps may have been captured)."""
+        """Floats of the line sweep's partial sinograms, the most any subset or the full angle set needs (so that the
+        workspace does not grow within a run, whose steps may have been captured)."""
         key = (getattr(self, "_subsets_version", 0), self.radon_variant.get("fwd_lines"), n_angles, kn)
         cap = self._lines_caps.get(key)
         if cap is None:
-            sets = [(tab, n_angles)]
+            sets = [(tab, n_angles), (self._tables_full, self.N_Omega)]
             if self.omega_subsets is not None and self._sub_tables is not None:
                 sets += [(t, len(s)) for t, s in zip(self._sub_tables, self.omega_subsets)]
-            cap = max(self._lines_variant(t, kn)[0] * n * self.My * kn for t, n in sets)
+            split = [(self._lines_variant(t, kn)[0], n) for t, n in sets]
+            cap = max(ns * n * self.My * kn if ns > 1 else 0 for ns, n in split)
             self._lines_caps = {**self._lines_caps, key: cap} if len(self._lines_caps) < 64 else {key: cap}
         return cap
 

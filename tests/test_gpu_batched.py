@@ -134,3 +134,37 @@ def test_batched_graph_replay_matches_eager():
             torch.cuda.synchronize()
         res.append(bat.xk.clone())
     assert torch.equal(res[0], res[1])
+
+
+def test_batched_graphs_follow_the_workspace():
+    """Images whose forward projection splits its lines over workgroups (partial sums in the operator's workspace), with
+    full forwards between replayed steps: the workspace serves the full angle set from the start, the captured steps are
+    dropped when it is replaced, and the iterates equal the eager ones bit for bit."""
+    import torch
+    from diffractom_amd.batched import BatchedSPDHGPoisson
+    print("case batched graphs workspace", flush=True)
+    c = cfg(nx=84, ny=83, my=87, n_omega=20, n_eta=12, angle_range=(0, 180), cor=0.3)
+    res = []
+    for graphs in (False, True):
+        ops = [build(c, K=K, pf_mode="sparse", pf_precision="bf16_residual", oracle=False)[0] for K in (12, 20)]
+        bs = [torch.poisson(torch.full(op.data_shape, 20.0), generator=torch.Generator().manual_seed(i)).cuda()
+              for i, op in enumerate(ops)]
+        bat = BatchedSPDHGPoisson(ops, subsets=3, seed=3, graphs=graphs)
+        bat.start(None, bs)
+        o0 = ops[0]
+        assert o0._fwd_kernel(o0._tables(0), 6, bat.Kc) == "lines" and o0._lines_variant(o0._tables(0), bat.Kc)[0] > 1
+        if graphs:
+            assert bat.capture_all() == 6
+        gen = o0.scratch_generation
+        for _ in range(3):
+            bat.advance(4)
+            torch.cuda.synchronize()
+            bat.step(None, full_forward=True)
+            assert o0.scratch_generation == gen
+        o0._t_buf(o0._t_buf_t.numel() + 64)
+        bat.advance(1)
+        assert not bat._graph_cache
+        bat.advance(9)
+        torch.cuda.synchronize()
+        res.append(bat.xk.clone())
+    assert torch.equal(res[0], res[1])
