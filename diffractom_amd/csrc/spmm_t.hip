@@ -15,11 +15,18 @@
 // its operand is one contiguous 16-byte read per lane. Four entries cost 1 add, 4 NB FMAs and NB LDS reads for 64 NB
 // detector positions; with an entry per wave-instruction (two v_readlane, an add and 4-byte reads each) they cost 4
 // times (3 + NB), and that issue rate bounded the kernel: 9899 orientations x 180 angles x 900 segments x 103 rows, 6.2 %
-// fill (9.9e7 entries), forward 2.59 -> 1.63 ms with its split and transposes, adjoint 1.32 ms. VALU issue (82 % of the
-// cycles) still bounds it: a third of it entries, the rest the visits, their rounding to 4 entries and the staging. Rows whose entries run out in a chunk before the others' of
-// their quad read a zero operand. The first two windows of a visit are loaded one visit ahead. Summation follows the CSR
-// order, as in the row-per-thread kernels.
+// fill (9.9e7 entries), forward with its split in two and transposes 2.47 -> 1.77 ms, adjoint 2.05 -> 1.30. VALU issue
+// still bounds it: a third of it entries, the rest the visits, their rounding to 4 entries and the staging. Rows whose
+// entries run out in a chunk before the others' of their quad read a zero operand. The first two windows of a visit are
+// loaded one visit ahead.
+//
+// Summation. Products into the transposed output (the forward: long rows of orientations) sum a row's entries of a chunk
+// apart, in A interleaved sums, and add them to the row's sum, up to 192 detector positions: the FP32 chain is a chunk's
+// entries / A and then the chunks, whatever the number of ranges (one chain instead: 1500 orientations in one range
+// 1.4e-7 from 64 bits, so 4.8e-8, 3 % of the time). Otherwise (the adjoint: rows of segments; above 192 positions, where
+// the registers leave no room for sums apart) a row is one chain in CSR order, as in the row-per-thread kernels.
 #include <algorithm>
+#include <type_traits>
 
 #include "dfm_common.h"
 
@@ -50,18 +57,20 @@ __device__ __forceinline__ void entry_load(const char* lds, int off, int lane16,
 #pragma unroll
   for (int h = 0; h < NB; ++h) x[h] = *reinterpret_cast<const f32x4*>(p + 256 * h);
 }
-template <int K, int NB>
+template <int K, int NB, bool FIRST>
 __device__ __forceinline__ void entry_fma(int vb, const f32x4 (&x)[NB], f32x4 (&acc)[NB]) {
   const float v = __int_as_float(bcast16<K>(vb));
 #pragma unroll
   for (int h = 0; h < NB; ++h)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) acc[h][e] += v * x[h][e];
+    for (int e = 0; e < 4; ++e) acc[h][e] = FIRST ? v * x[h][e] : acc[h][e] + v * x[h][e];
 }
 
-// entries K .. 15 of the windows while fewer than `steps` are done, U operand rows in flight
-template <int K, int U, int NB>
-__device__ __forceinline__ void window(const char* lds, int off, int vb, int lane16, int steps, f32x4 (&acc)[NB]) {
+// entries K .. 15 of the windows while fewer than `steps` are done, U operand rows in flight; entry t goes to sum t % A.
+// FIRST: the sums start with the first A entries
+template <int K, int U, int A, int NB, bool FIRST>
+__device__ __forceinline__ void window(const char* lds, int off, int vb, int lane16, int steps, f32x4 (&acc)[A][NB]) {
+  static_assert(U % A == 0, "a group of U entries starts every sum");
   if constexpr (K < 16) {
     if (steps <= K) return;                                  // uniform
     f32x4 x[U][NB];
@@ -72,13 +81,13 @@ __device__ __forceinline__ void window(const char* lds, int off, int vb, int lan
       entry_load<K + 3, NB>(lds, off, lane16, x[3]);
     }
     __builtin_amdgcn_sched_barrier(0);
-    entry_fma<K, NB>(vb, x[0], acc);
-    if constexpr (U > 1) entry_fma<K + 1, NB>(vb, x[1], acc);
+    entry_fma<K, NB, FIRST>(vb, x[0], acc[0]);
+    if constexpr (U > 1) entry_fma<K + 1, NB, FIRST && (A > 1)>(vb, x[1], acc[1 % A]);
     if constexpr (U > 2) {
-      entry_fma<K + 2, NB>(vb, x[2], acc);
-      entry_fma<K + 3, NB>(vb, x[3], acc);
+      entry_fma<K + 2, NB, FIRST && (A > 2)>(vb, x[2], acc[2 % A]);
+      entry_fma<K + 3, NB, FIRST && (A > 2)>(vb, x[3], acc[3 % A]);
     }
-    window<K + U, U, NB>(lds, off, vb, lane16, steps, acc);
+    window<K + U, U, A, NB, false>(lds, off, vb, lane16, steps, acc);
   }
 }
 
@@ -88,7 +97,8 @@ __device__ __forceinline__ int window_steps(unsigned long long m) {
   return __popc((f | f >> 16) & 0xffffu);
 }
 
-template <int R, int NB, int U>
+// A > 0: a row's entries of a chunk are summed apart (A interleaved sums), then added to the row's sum; 0: one chain
+template <int R, int NB, int U, int A>
 __global__ void __launch_bounds__(1024) spmm_t_kernel(const float* __restrict__ inT, const int* __restrict__ row_ptr,
                                                       const uint16_t* __restrict__ col, const float* __restrict__ val,
                                                       float* __restrict__ outT, const int* __restrict__ omegas,
@@ -133,11 +143,11 @@ __global__ void __launch_bounds__(1024) spmm_t_kernel(const float* __restrict__ 
       cur[i] = lo;
     }
   }
-  f32x4 acc[R][NB];
+  f32x4 acc[R][1][NB];
 #pragma unroll
   for (int i = 0; i < R; ++i)
 #pragma unroll
-    for (int h = 0; h < NB; ++h) acc[i][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int h = 0; h < NB; ++h) acc[i][0][h] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // window entry `cu + l16` of a row ending at en (past the end: a repeated entry, not counted)
   auto fetch = [&](int cu, int en, int& c, float& v) {
@@ -225,24 +235,44 @@ __global__ void __launch_bounds__(1024) spmm_t_kernel(const float* __restrict__ 
       fetch(cur[i + 1 < R ? i + 1 : 0], end[i + 1 < R ? i + 1 : 0], pc0, pv0);
       fetch(cur[i + 1 < R ? i + 1 : 0] + 16, end[i + 1 < R ? i + 1 : 0], pc1, pv1);
       __builtin_amdgcn_sched_barrier(0);
-      window<0, U, NB>(lds, off0, vb0, lane16, window_steps(m0), acc[i]);
-      if (m1) window<0, U, NB>(lds, off1, vb1, lane16, window_steps(m1), acc[i]);
-      bool more = __any(n == 32);
-      while (more) {                                         // a row with more than 32 entries in the chunk
-        int c;
-        float v;
-        fetch(cur[i], end[i], c, v);
-        const bool in = cur[i] + l16 < end[i] && c < c1;
-        const unsigned long long m = __ballot(in);
-        window<0, U, NB>(lds, in ? row_off(c - c0) : zoff, in ? __float_as_int(v) : 0, lane16, window_steps(m),
-                         acc[i]);
-        const int nn = __popc((unsigned)(m >> shift) & 0xffffu);
-        cur[i] += nn;
-        more = __any(nn == 16);
-        if (R == 1) {                                        // the next visit is this row's
-          fetch(cur[0], end[0], pc0, pv0);
-          fetch(cur[0] + 16, end[0], pc1, pv1);
+      // the visit's windows into p; a row with more than 32 entries in the chunk has more of them
+      auto windows = [&](auto first, auto& p) {
+        constexpr int NA = sizeof(p) / sizeof(p[0]);
+        window<0, U, NA, NB, decltype(first)::value>(lds, off0, vb0, lane16, window_steps(m0), p);
+        if (m1) window<0, U, NA, NB, false>(lds, off1, vb1, lane16, window_steps(m1), p);
+        bool more = __any(n == 32);
+        while (more) {
+          int c;
+          float v;
+          fetch(cur[i], end[i], c, v);
+          const bool in = cur[i] + l16 < end[i] && c < c1;
+          const unsigned long long m = __ballot(in);
+          window<0, U, NA, NB, false>(lds, in ? row_off(c - c0) : zoff, in ? __float_as_int(v) : 0, lane16,
+                                      window_steps(m), p);
+          const int nn = __popc((unsigned)(m >> shift) & 0xffffu);
+          cur[i] += nn;
+          more = __any(nn == 16);
+          if (R == 1) {                                      // the next visit is this row's
+            fetch(cur[0], end[0], pc0, pv0);
+            fetch(cur[0] + 16, end[0], pc1, pv1);
+          }
         }
+      };
+      if constexpr (A > 0) {
+        if (m0) {                                            // uniform
+          f32x4 p[A][NB];
+          windows(std::true_type{}, p);
+#pragma unroll
+          for (int s = A / 2; s > 0; s /= 2)
+#pragma unroll
+            for (int q = 0; q < s; ++q)
+#pragma unroll
+              for (int h = 0; h < NB; ++h) p[q][h] += p[q + s][h];
+#pragma unroll
+          for (int h = 0; h < NB; ++h) acc[i][0][h] += p[0][h];
+        }
+      } else {
+        windows(std::false_type{}, acc[i]);
       }
     }
   }
@@ -259,7 +289,7 @@ __global__ void __launch_bounds__(1024) spmm_t_kernel(const float* __restrict__ 
 #pragma unroll
       for (int i = 0; i < R; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) lin[(4 * l16 + e) * RW + rw0 + 4 * i] = alpha * acc[i][h][e];
+        for (int e = 0; e < 4; ++e) lin[(4 * l16 + e) * RW + rw0 + 4 * i] = alpha * acc[i][0][h][e];
       __syncthreads();
       if (row < rows_out)
         for (int yl = threadIdx.x / RB; yl < 64 && 64 * h + yl < my; yl += SPT_WAVES * 64 / RB)
@@ -276,7 +306,7 @@ __global__ void __launch_bounds__(1024) spmm_t_kernel(const float* __restrict__ 
       for (int h = 0; h < NB; ++h) {
         const int y = 64 * h + 4 * l16;
         float* d = dst + (int64_t)row * ys_out + y;
-        const f32x4 v = alpha * acc[i][h];
+        const f32x4 v = alpha * acc[i][0][h];
         if (vec_out && y + 3 < my) {
           *reinterpret_cast<f32x4*>(d) = v;
         } else {
@@ -330,9 +360,14 @@ void launch_spmm_t(dim3 grid, size_t lds, hipStream_t st, const float* inT, cons
                    int rows_out, int compact, float alpha, int cspan, int kc, int n_angles, int64_t in_ld,
                    int64_t out_ld, int ys_out) {
   const int vec_out = ys_out % 4 == 0 && (uintptr_t)outT % 16 == 0;
-  hipLaunchKernelGGL((spmm_t_kernel<R, NB, (NB <= 2 ? 4 : NB <= 4 ? 2 : 1)>), grid, dim3(SPT_WAVES * 64), lds, st,
-                     inT, row_ptr, col, val, outT, omegas, my, ys, ncols, nrows, rows_out, compact, alpha, cspan, kc,
-                     n_angles, in_ld, out_ld, ys_out, vec_out);
+  constexpr int U = NB <= 2 ? 4 : NB <= 4 ? 2 : 1, A = NB == 1 ? 4 : NB <= 3 ? 2 : 0;
+#define DFM_SPT_A(AA)                                                                                               \
+  hipLaunchKernelGGL((spmm_t_kernel<R, NB, U, AA>), grid, dim3(SPT_WAVES * 64), lds, st, inT, row_ptr, col, val, outT, \
+                     omegas, my, ys, ncols, nrows, rows_out, compact, alpha, cspan, kc, n_angles, in_ld, out_ld,    \
+                     ys_out, vec_out)
+  if (out_ld) DFM_SPT_A(0);
+  else DFM_SPT_A(A);
+#undef DFM_SPT_A
 }
 
 // row quads per wave: 4 (256 rows a workgroup), 2 where the accumulators of more than 128 detector positions leave no

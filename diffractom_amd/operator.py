@@ -1475,19 +1475,29 @@ class SinglePhaseForwardOperator:
         return [p[o:o + int(z)] for o, z in zip(offs, sizes)]
 
     def _tsplit(self, n_ang, kb):
-        """Orientation split of the transposed forward: 64 workgroups of the most rows (the kernel takes fewer rows in
-        each, down to a quarter, where they are fewer than 128; a workgroup's LDS fills a CU), in ranges of 256
-        orientations or more, for every split writes and adds up a partial result (us for a split of 1 / 2 / 4, 900
-        segments x 103 rows: 9899 orientations x 180 angles 1630 / 1724 / 1905, 1500 x 18 64 / 66 / 72, 543 x 23 25 / 27
-        / 39). Below 1024 workgroups, ranges of at most 5120 orientations, which bounds the FP32 chains: at 9899 x 180 one
-        range is 5 % faster and twice as far from 64 bits (3.8e-7 against 2.0e-7)."""
+        """Orientation split of the transposed forward. Up to 192 detector positions: 64 workgroups of the most rows (the
+        kernel takes fewer rows in each, down to a quarter, where they are fewer than 128; a workgroup's LDS fills a
+        CU), in ranges of 256 orientations or more, for every split writes and adds up a partial result (us for a split
+        of 1 / 2 / 4, 900 segments x 103 rows: 9899 orientations x 180 angles 1675 / 1773 / 1964, 1500 x 18 63 / 65 /
+        71, 543 x 23 24 / 26 / 39). Below 1024 workgroups, ranges of at most 5 LDS chunks (4 above 128 positions): the
+        kernel sums every chunk apart, so the number of chunks is the length of the FP32 chain that is left. These lines
+        keep the error against 64 bits where the finest split (1024 workgroups, ranges of 128 orientations or more) has
+        it: 900 segments x 103 rows, this / the finest / one chain: 333 orientations x 50 angles 6.3e-8 / 6.3e-8 /
+        1.0e-7, 543 x 23 3.9e-8 / 3.8e-8 / 3.7e-8 (0.6 % fill), 1500 x 18 4.8e-8 / 5.8e-8 / 1.4e-7, 9899 x 180 5.9e-8 /
+        1.9e-7 / 3.8e-7; in a model of the sums over 0.6 to 20 % fill and 400 to 9899 orientations 0.35 to 1.09 times
+        it. The finest split is taken above 192 positions, where the registers leave no room for sums apart."""
         v = self.csr_variant.get("tsplit", "auto")
         if v != "auto":
             return int(max(1, min(int(v), max(kb, 1))))
+        nb = -(-self.My // 64)
+        most = -(-1024 // (-(-self.N_seg // self._t_rows) * n_ang))
+        if nb > 3:
+            return int(max(1, min(64, most, kb // 128)))
         if kb < 512:
             return 1
         wgs = -(-self.N_seg // self._t_rows) * n_ang
-        ns = max(min(-(-64 // wgs), max(kb // 256, 1)), min(-(-1024 // wgs), -(-kb // 5120)))
+        chunks = -(-kb // (40960 // (64 * nb) - 1))          # of the kernel's LDS
+        ns = max(min(-(-64 // wgs), kb // 256), min(most, -(-chunks // (5 if nb <= 2 else 4))))
         return int(max(1, min(64, ns)))
 
     def _spmm_t_forward(self, b, sb, om, n_ang, sino, data, accumulate):
