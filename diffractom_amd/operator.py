@@ -1060,18 +1060,20 @@ class SinglePhaseForwardOperator:
 
     def _lines_variant(self, tab, kn):
         """(line ranges, duplicated layout) of the line sweep: radon_variant["fwd_lines"] (ranges + 128 for the
-        duplicated layout) if set by hand or by autotune, else by size. The duplicated layout while two workgroups of
+        duplicated layout, 0 ranges: by size) if set by hand or by autotune, which sets the layout alone (the ranges
+        that suit one subset are too many for all angles), else by size. The duplicated layout while two workgroups of
         it fit a CU's LDS (128 pixels: 99 x 99 x 29760 x 18 angles 0.82 against 0.89 ms; 256 pixels, one workgroup: 1.62
         against 1.20). With fewer workgroups than CUs the lines are split for two workgroups per CU, in ranges of 8
         lines or more and at most 12 (99 x 99 x 18 angles: 576 orientations 109 -> 46 us, 2048 117 -> 92 us; 5056, 316
         workgroups, 178 -> 198)."""
-        v = self.radon_variant.get("fwd_lines")
-        if v is not None:
-            return int(v) % 128, int(v) // 128
         n = max(self.Nx, self.Ny)
+        v = self.radon_variant.get("fwd_lines")
+        dup = int(n <= 128) if v is None else int(v) // 128
+        if v is not None and int(v) % 128:
+            return int(v) % 128, dup
         wgs = -(-kn // 32) * tab["sweep_grp_p"].shape[0]
         nsplit = 1 if wgs >= 256 else max(1, min((512 + wgs // 2) // wgs, n // 8, 12))
-        return nsplit, int(n <= 128)
+        return nsplit, dup
 
     def _lines_part(self, tab, n_angles, kn):
         """Floats of the line sweep's partial sinograms, the most any subset or the full angle set needs (so that the
@@ -1162,10 +1164,7 @@ class SinglePhaseForwardOperator:
             sl = _lib.load().dfm_radon_sweep_lines(self.Nx, self.Ny)
             if tab["pairs_ok"] and max(self.Nx, self.Ny) <= 256:
                 # the line sweep first: the fastest at every measured configuration but small images
-                rv["fwd_lines"] = None
-                nsplit, _ = self._lines_variant(tab, kn)
-                cands.update({f"lines:{n}" + "+dup" * d: ("lines", n + 128 * d) for n in sorted({nsplit, 1})
-                              for d in (1, 0)})
+                cands.update({"lines" + "+dup" * d: ("lines", 128 * d) for d in (1, 0)})
             if sl and self.My <= 1024:         # 1024 rays per workgroup (512 for the 64-orientation form)
                 cands.update({f"sweep:{n}": ("sweep", n) for n in (4,) if n <= sl})
                 ln = max(self.Nx, self.Ny)

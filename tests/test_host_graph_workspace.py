@@ -106,3 +106,31 @@ def test_partial_sinograms_are_sized_for_every_angle_set(n, my, n_omega, M, kn):
     most = max(need(t, na) for t, na in sets)
     for t, na in sets:
         assert op._lines_part(t, na, kn) == most
+
+
+def test_tuned_line_sweep_keeps_the_rule_for_other_launches():
+    """Autotuning on a subset that splits its lines leaves the number of ranges of every other launch to the rule."""
+    from diffractom_amd import _lib
+    if not _lib.LIB_PATH.exists():
+        pytest.skip("the library is not built")
+    n, my, n_omega, M, kn = 99, 103, 180, 10, 576
+    op = object.__new__(SinglePhaseForwardOperator)
+    op.Nx = op.Ny = n
+    op.My, op.N_Omega, op._lines_caps, op.fourier, op.radon_bands = my, n_omega, {}, None, 1
+    op.radon_variant = {"fwd": 8 + 256, "bwd": None, "fwd_kernel": None, "bwd_kernel": "table"}
+
+    def tables(na):
+        return {"sweep_grp_p": np.zeros((-(-na // 9), 1)), "pairs_ok": True, "mfma_ok": True, "tbase8": torch.zeros(2)}
+    op._tables_full, op.omega_subsets = tables(n_omega), [np.arange(m, n_omega, M) for m in range(M)]
+    op._sub_tables = [tables(len(s)) for s in op.omega_subsets]
+    sub, full = op._sub_tables[0], op._tables_full
+    rule = {k: op._lines_variant(full, k) for k in (64, kn, 9920)}
+    assert op._lines_variant(sub, kn)[0] > 1 and rule[kn][0] < op._lines_variant(sub, kn)[0]
+    op._angle_set = lambda m: (len(op.omega_subsets[m]), None, None, None)
+    op._radon_backward = lambda *a, **k: 1.0
+    # the line sweep is the fastest, the more ranges the better
+    op._radon_forward = lambda *a: (1.0 / op._lines_variant(sub, kn)[0] if op.radon_variant["fwd_kernel"] == "lines"
+                                    else 9.0)
+    op.tune_projector(0, None, kn, 0, kn, None, None, None, None, lambda f: f())
+    assert op.radon_variant["fwd_kernel"] == "lines"
+    assert {k: op._lines_variant(full, k)[0] for k in rule} == {k: r[0] for k, r in rule.items()}
