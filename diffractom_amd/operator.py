@@ -1051,10 +1051,14 @@ class SinglePhaseForwardOperator:
         angle) triples on (us, against the table, launches back to back: 99 x 99 x 64 x 18 angles 22 / 37, 88 x 88 x
         2048 x 6 36 / 56, 64 x 64 x 2048 x 60 68 / 144, 99 x 99 x 9920 x 180 2020 / 4830). Below that its second launch
         and its chain of lines cost what they save or more (72 x 72 x 512 x 18 31 / 26, 64 x 64 x 6016 x 6 68 / 58, 32 x
-        32 x 512 x 18 17 / 9). Otherwise the table, in bands for large images."""
-        n = max(self.Nx, self.Ny)
-        if (n > 80 or self.Nx * self.Ny * n_angles * kn >= 150_000_000) and tab is not None and n <= 256 and \
-                tab["pairs_ok"]:
+        32 x 512 x 18 17 / 9). Otherwise the table, in bands for large images. Half of the angles sweep the columns, so
+        the walk goes with the longer side and the table's work with the pixels: images of less than 64 pixels on one
+        side and twice that on the other take the table (x 2048 orientations x 18 angles: 256 x 8 335 / 47, 128 x 16 119
+        / 35, 256 x 32 342 / 180, 128 x 51 122 / 97; 100 x 50 63 / 75, 200 x 64 201 / 264), and the triples count by
+        the sides' ratio squared (64 x 32 x 9920 x 18 130 / 101, x 90 336 / 461)."""
+        n, m = max(self.Nx, self.Ny), min(self.Nx, self.Ny)
+        if (n > 80 or self.Nx * self.Ny * n_angles * kn * m * m >= 150_000_000 * n * n) and (m >= 64 or 2 * m >= n) and \
+                tab is not None and n <= 256 and tab["pairs_ok"]:
             return "lines"
         return "band" if self.radon_bands >= 4 else "table"
 
@@ -1064,7 +1068,7 @@ class SinglePhaseForwardOperator:
         that suit one subset are too many for all angles), else by size. The duplicated layout while two workgroups of
         it fit a CU's LDS (128 pixels: 99 x 99 x 29760 x 18 angles 0.82 against 0.89 ms; 256 pixels, one workgroup: 1.62
         against 1.20). With fewer workgroups than CUs the lines are split for two workgroups per CU, in ranges of 8
-        lines or more and at most 12 (99 x 99 x 18 angles: 576 orientations 109 -> 46 us, 2048 117 -> 92 us; 5056, 316
+        lines or more along the longer side and at most 12 (99 x 99 x 18 angles: 576 orientations 109 -> 46 us, 2048 117 -> 92 us; 5056, 316
         workgroups, 178 -> 198)."""
         n = max(self.Nx, self.Ny)
         v = self.radon_variant.get("fwd_lines")
