@@ -1465,14 +1465,16 @@ class SinglePhaseForwardOperator:
         return -(-self.My // 4) * 4
 
     def _t_buf(self, *sizes):
-        """Views of one reusable workspace, each starting 256-byte aligned."""
+        """Views of one reusable workspace, each starting 256-byte aligned. It is allocated for the stream that the
+        operator launches on, so that its memory is not handed out again, when it grows, before that stream is done."""
         offs, n = [], 0
         for z in sizes:
             offs.append(n)
             n += -(-int(z) // 64) * 64
         p = getattr(self, "_t_buf_t", None)
         if p is None or p.numel() < n:
-            p = torch.empty(n, dtype=torch.float32, device=self.device)
+            with torch.cuda.stream(self.queue):              # (None: the current stream)
+                p = torch.empty(n, dtype=torch.float32, device=self.device)
             self._t_buf_t = p
             self.scratch_generation = getattr(self, "scratch_generation", 0) + 1
         return [p[o:o + int(z)] for o, z in zip(offs, sizes)]
@@ -1567,7 +1569,8 @@ class SinglePhaseForwardOperator:
     def _mfma_part(self, n):
         p = getattr(self, "_mfma_part_buf", None)
         if p is None or p.numel() < n:
-            p = torch.empty(n, dtype=torch.float32, device=self.device)
+            with torch.cuda.stream(self.queue):              # as _t_buf
+                p = torch.empty(n, dtype=torch.float32, device=self.device)
             self._mfma_part_buf = p
             self.scratch_generation = getattr(self, "scratch_generation", 0) + 1
         return p

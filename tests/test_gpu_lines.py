@@ -107,3 +107,25 @@ def test_subsets_of_different_sizes_under_graphs(K):
         torch.cuda.synchronize()
         out.append(sol.xk.cpu().numpy())
     assert np.array_equal(out[0], out[1])
+
+
+def test_workspace_belongs_to_the_operators_stream():
+    """The partial sums' workspaces of an operator with a stream of its own come from that stream's memory, and its
+    products equal those on the current stream."""
+    import torch
+    print("case lines workspace stream", flush=True)
+    out = []
+    for queue in (None, torch.cuda.Stream()):
+        op, _, _ = build(cfg(nx=84, ny=83, my=87, n_omega=12, n_eta=36), K=800, pf_mode="sparse",
+                         pf_precision="bf16_residual", oracle=False)
+        op.queue = queue
+        x = torch.rand(op.coeff_shape, generator=torch.Generator().manual_seed(3)).cuda()
+        d = torch.zeros(op.data_shape, device="cuda")
+        torch.cuda.synchronize()
+        op.direct_cl(x, d)
+        torch.cuda.synchronize()
+        out.append(d.cpu().numpy())
+        for buf in (op._t_buf_t, op._mfma_part_buf):
+            seg = [s for s in torch.cuda.memory_snapshot() if s["address"] <= buf.data_ptr() < s["address"] + s["total_size"]]
+            assert len(seg) == 1 and seg[0]["stream"] == (0 if queue is None else queue.cuda_stream)
+    assert np.array_equal(out[0], out[1])
