@@ -182,10 +182,12 @@ __global__ void __launch_bounds__(TH, 4) radon_forward_lines_kernel(
     }
   }
   // ---- an infinite or NaN pixel must reach the rays with a weight on it and no others: where a sum is not finite, it is
-  // made again from memory without the products with zero weights
+  // made again from memory without the products with zero weights (of quads beyond the last, whose LDS nothing wrote,
+  // the sums mean nothing)
   float nf = 0.f;
 #pragma unroll
   for (int qq = 0; qq < CQ; ++qq) {
+    if (q0 + ((qq + rot) & (CQ - 1)) >= k4_n) continue;
     nf = fmaf(accL[qq].x, 0.f, fmaf(accL[qq].y, 0.f, fmaf(accL[qq].z, 0.f, fmaf(accL[qq].w, 0.f, nf))));
     nf = fmaf(accR[qq].x, 0.f, fmaf(accR[qq].y, 0.f, fmaf(accR[qq].z, 0.f, fmaf(accR[qq].w, 0.f, nf))));
   }

@@ -129,3 +129,26 @@ def test_workspace_belongs_to_the_operators_stream():
             seg = [s for s in torch.cuda.memory_snapshot() if s["address"] <= buf.data_ptr() < s["address"] + s["total_size"]]
             assert len(seg) == 1 and seg[0]["stream"] == (0 if queue is None else queue.cuda_stream)
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("koff,kn", [(0, 4), (8, 20), (32, 32), (12, 52)])
+def test_column_ranges(koff, kn):
+    """Column ranges that fill a part of a block of 32 orientations: the columns of the whole product, nothing beyond."""
+    import torch
+    from diffractom_amd import _lib
+    print(f"case lines columns koff={koff} kn={kn}", flush=True)
+    op, img = _setup(40, 33, 43, 7, 64)
+    whole = _sino(op, img, 1, 1)
+    t, g = op._tables_full, op._tables_full["sweep_grp_p"]
+    for nsplit, dup in ((1, 1), (3, 0)):
+        out = torch.full((op.N_Omega * op.My, 64), 7.0, device="cuda")
+        part = torch.empty(nsplit * out.numel(), device="cuda")
+        _lib.call("dfm_radon_forward_lines", _lib.ptr(img), _lib.ptr(out), _lib.ptr(part), _lib.ptr(t["sweep_geo"]),
+                  _lib.ptr(g), _lib.ptr(t["sweep_gcls_p"]), g.shape[0], g.shape[1], op.N_Omega, op.My, op.Nx, op.Ny,
+                  op.K_stride, koff, kn, 64, nsplit, dup, op._stream())
+        got = out.cpu().numpy()
+        assert np.all(got[:, kn:] == 7.0)
+        ref = whole[:, koff:koff + kn]
+        # split lines: the sums' order differs, 6 roundings per line on terms of one magnitude
+        tol = 0.0 if nsplit == 1 else (6 * 40 + 2) * 2.0 ** -24 * float(img.abs().max()) * 40 * 4 * op.radon_scale
+        assert np.abs(got[:, :kn] - ref).max() <= tol
