@@ -266,28 +266,33 @@ def test_block_workgroup_sizes_agree(mode, precision):
         assert np.array_equal(u, v)
 
 
-@pytest.mark.parametrize("my", [103, 90])
-@pytest.mark.parametrize("mode,precision", [("sparse", "bf16_residual"), ("sparse", "fp16"), ("generated", "fp16")])
-def test_block_fixed_tile_count_agrees(mode, precision, my):
-    """The 4-wave block products with the y-tile count compiled in (7 tiles at 103 detector rows, 6 at 90) give the
-    run-time count's results bit for bit (the same tiles, chunks and accumulation order)."""
+@pytest.mark.parametrize("my", [103, 90, 131, 128, 40, 17])
+@pytest.mark.parametrize("precision", ["bf16", "bf16_residual", "fp16"])
+def test_block_fixed_tile_count_agrees(precision, my):
+    """The 4-wave grouped block products with the y-tile count compiled in (7 tiles at 103 detector rows, 6 at 90, two
+    groups of 5 at 131, 8 at 128, 4 at 40, 2 at 17) give the results of the form with a run-time count bit for bit (the
+    same tiles, chunks and accumulation order)."""
     import torch
-    print(f"case block fixed tile count {mode} {precision} my={my}", flush=True)
+    from diffractom_amd import _lib
+    from diffractom_amd.batched import BatchedSPDHGPoisson, _blk_y_tiling
+    print(f"case block fixed tile count {precision} my={my}", flush=True)
     c = cfg(nx=12, ny=12, my=my, n_omega=12, angle_range=(0, 180), cor=0.3)
-    op, _, _ = build(c, K=300, pf_mode=mode, pf_precision=precision, oracle=False)
-    op.set_omega_subsets(3)
-    x, y = _inputs(op, 7)
-    xt, yt = torch.from_numpy(x).cuda(), torch.from_numpy(y).cuda()
-    res = []
-    for fixed in (False, True):
-        op.blk_variant.update(fwd_wg=4, adj_wg=4, fwd_fixed=fixed, adj_fixed=fixed)
-        out = []
-        for sub in (None, 1):
-            d = torch.zeros(op.data_shape, device="cuda")
-            a = torch.zeros(op.coeff_shape, device="cuda")
-            op.direct_cl(xt, d, subset=sub)
-            op.adjoint_cl(yt, a, subset=sub)
-            out += [d.cpu().numpy(), a.cpu().numpy()]
-        res.append(out)
-    for u, v in zip(*res):
-        assert np.array_equal(u, v)
+    ops = [build(c, K=K, pf_mode="sparse", pf_precision=precision, oracle=False)[0] for K in (300, 45)]
+    bat = BatchedSPDHGPoisson(ops, subsets=3)
+    bat.start(None, [torch.full(op.data_shape, 20.0, device="cuda") for op in ops])
+    mt_n, n_yg = _blk_y_tiling(my, bat.Kc)
+    assert mt_n == {103: 7, 90: 6, 131: 5, 128: 8, 40: 4, 17: 2}[my]
+    g = torch.Generator(device="cuda").manual_seed(my)
+    sino, data = (torch.rand(t.shape, generator=g, device="cuda") - 0.3 for t in (bat.sino, bat.D))
+    mode = ops[0]._blk_mode("fwd") & 15
+    for sub in (None, 1):
+        for forward, src, dst in ((True, sino, bat.D), (False, data, bat.sino)):
+            buf, wgm, n_wg = bat._group(forward, sub)
+            out = []
+            for count in (0, mt_n):
+                (bat.sino if forward else bat.D).copy_(src)
+                dst.fill_(7.0)
+                _lib.call("dfm_pfblk_grouped", int(forward), _lib.ptr(buf), _lib.ptr(wgm), n_wg, mode | count << 8,
+                          ops[0]._stream())
+                out.append(dst.cpu().numpy())
+            assert np.array_equal(*out) and not np.all(out[0] == 7.0)
