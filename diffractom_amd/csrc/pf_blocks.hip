@@ -17,10 +17,12 @@
 // entries, read back in operand order: lane l holds 8 consecutive contraction indices of column l % 16), while the
 // workgroup's four waves share the y-side operand chunk (FP32 from HBM, split into bf16 hi/lo or scaled to fp16 in
 // LDS, double buffered). What bounds it: the chunk's latency (loads, LDS expansion, barrier), so the loads run two
-// chunks ahead, in code without branches around them, and the tile loops have compiled counts. 18 angles x 103 rows x
-// 29,713 orientations x 1,440 segments (65 GFLOP of tiles, 0.28 GB of PF), loads in branches / as here: residual
-// forward 511 / 387 us, adjoint 389 / 341; fp16 557 / 411 and 445 / 430; 90 angles x 131 rows x 5,000 x 1,440,
-// residual: 722 / 520 and 557 / 459. v_mfma_f32_16x16x32_{bf16,f16}, FP32 accumulation; the residual mode adds hi*hi + hi*lo +
+// chunks ahead, in code without branches around them, and the tile loops have compiled counts with the operands read a few
+// tiles ahead. 18 angles x 103 rows x 29,713 orientations x 900 segments (65 GFLOP of tiles, 0.28 GB of PF), loads in
+// branches and run-time counts / as here: residual forward 517 / 375 us, adjoint 407 / 335; fp16 834 / 413 and 619 / 435;
+// bf16 447 / 305 and 343 / 292; 90 angles x 131 rows x 5,000 x 900, residual: 718 / 519 and 554 / 465; 18 angles x 103
+// rows x 12, the one chunk with fewer columns: 10.8 / 10.6 and 46 / 33.
+// v_mfma_f32_16x16x32_{bf16,f16}, FP32 accumulation; the residual mode adds hi*hi + hi*lo +
 // lo*hi (lo*lo, 2^-16 relative, dropped). In the fp16 mode every (row, chunk) of the y-side operand is scaled by a
 // power of two that puts its largest magnitude at 2^14 (fp16 keeps 11 significant bits from 2^-14 up), and the
 // product of the chunk is scaled back before it is added to the FP32 accumulator; the ring scale of the PF is
@@ -208,11 +210,12 @@ __device__ __forceinline__ void blk_pf_body(const BlkArgs& p, int64_t w) {
   const int src_n = FWD ? p.kb : p.cp;
   const int c_full = src_n >> 5;                             // chunks with all 32 columns; at most one after them
   const int scol = ((tid & 63) >> 4) * 8;                    // the same for every slot of this thread
-  // the group's rows as a buffer (reads past its end give 0; they occur where there are fewer than 32 columns in all),
-  // and this thread's byte offsets in it
+  // the group's rows as a buffer that ends with the last row's last column (a dword past its end reads 0) and this
+  // thread's byte offsets in it. The chunk with fewer columns is read like the others, into the row after or past the
+  // end, and what is no column becomes 0 in store_lds
   const float* src = p.src + src_rows * src_stride;
   const __amdgpu_buffer_rsrc_t rsrc =
-      __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, (unsigned)rows * (unsigned)src_stride * 4u, 0x00027000);
+      __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, ((unsigned)(rows - 1) * src_stride + src_n) * 4u, 0x00027000);
   unsigned soff[NS];
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
@@ -221,9 +224,9 @@ __device__ __forceinline__ void blk_pf_body(const BlkArgs& p, int64_t w) {
     soff[i] = ((unsigned)y * (unsigned)src_stride + scol) * 4u;
   }
   typedef unsigned u4 __attribute__((ext_vector_type(4)));
-  // the rows of a full chunk (chunks beyond the range, or the last one with fewer columns, repeat the last full one)
+  // the rows of chunk c (beyond the range: of its last one)
   auto load_raw = [&](int c, float (&raw)[NS][8]) {
-    const int cbyte = max(min(min(c, c1 - 1), c_full - 1), 0) * 128;
+    const int cbyte = min(c, c1 - 1) * 128;
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
       const u4 u = __builtin_amdgcn_raw_buffer_load_b128(rsrc, soff[i], cbyte, 0);
@@ -248,11 +251,10 @@ __device__ __forceinline__ void blk_pf_body(const BlkArgs& p, int64_t w) {
 #pragma unroll
       for (int i = 0; i < NS; ++i)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) raw[i][e] = j0 + e < src_n ? src[(soff[i] >> 2) + c * 32 + e] : 0.f;
-#pragma unroll
-      for (int i = 0; i < NS; ++i)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) arrived(raw[i][e]);
+        for (int e = 0; e < 8; ++e) {
+          raw[i][e] = j0 + e < src_n ? raw[i][e] : 0.f;
+          arrived(raw[i][e]);                                // (keeps the selects in the branch)
+        }
     }
     if (F16 && !FWD) {
       // the ring scale of the PF folded into the data: column j = j0 + e, ring j % P
@@ -369,6 +371,32 @@ __device__ __forceinline__ void blk_pf_body(const BlkArgs& p, int64_t w) {
     for (int t = 0; t < 2; ++t) {
       bh[t] = b_frag[wv][0][t][lane];
       bl[t] = RES ? b_frag[wv][RES ? 1 : 0][t][lane] : zero8;
+    }
+    if constexpr (MTN > 0 && !F16) {
+      // the row tiles' operands a few tiles ahead (left to itself the compiler saves their registers and waits for each)
+      constexpr int D = RES ? 2 : 4;
+      s16x8 ah[MTN], al[RES ? MTN : 1];
+      auto read = [&](int mt) {
+        ah[mt] = a_hi[buf * MTB * 64 + mt * 64 + lane];
+        if (RES) al[mt] = a_lo[buf * MTB * 64 + mt * 64 + lane];
+      };
+#pragma unroll
+      for (int mt = 0; mt < (MTN < D ? MTN : D); ++mt) read(mt);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int mt = 0; mt < MTN; ++mt) {
+        if (mt + D < MTN) read(mt + D);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          acc[mt][t] = mma_bf16(ah[mt], bh[t], acc[mt][t]);
+          if (RES) {
+            acc[mt][t] = mma_bf16(ah[mt], bl[t], acc[mt][t]);
+            acc[mt][t] = mma_bf16(al[mt], bh[t], acc[mt][t]);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      return;
     }
 #pragma unroll
     for (int mt = 0; mt < MT_MAX; ++mt) {
@@ -495,8 +523,11 @@ __global__ __launch_bounds__(THREADS, MODE == MODE_F16 || MTN == 0 ? 2 : 3) void
 template <bool FWD, int MTN>
 void launch_blk_grouped_mt(const BlkArgs* descs, const int2* wg_map, int64_t n_map, int mode, hipStream_t st) {
   const dim3 grid((unsigned)((n_map + N_XCD - 1) / N_XCD * N_XCD)), block(THREADS);
+  // the residual adjoint of 8 tiles: compiled it needs 170 VGPRs, two workgroups a CU (4 slices of 40 to 2,000
+  // orientations x 18 angles x 128 rows: 74.5 us, with the run-time count and three workgroups 57.2)
+  constexpr int MTR = !FWD && MTN == 8 ? 0 : MTN;
   if (mode == MODE_BF16_RES)
-    hipLaunchKernelGGL((blk_pf_grouped_kernel<MODE_BF16_RES, FWD, MTN>), grid, block, 0, st, descs, wg_map, n_map);
+    hipLaunchKernelGGL((blk_pf_grouped_kernel<MODE_BF16_RES, FWD, MTR>), grid, block, 0, st, descs, wg_map, n_map);
   else if (mode == MODE_BF16)
     hipLaunchKernelGGL((blk_pf_grouped_kernel<MODE_BF16, FWD, MTN>), grid, block, 0, st, descs, wg_map, n_map);
   else
@@ -513,8 +544,9 @@ void launch_blk_wv(const BlkArgs& p, int mode, hipStream_t st) {
 }
 
 // y tiles per group that have a 4-wave form with the count compiled in: the tile loops carry no run-time bound, so a
-// chunk's LDS reads and MFMAs are one straight block, and three workgroups fit a CU (residual, 7 tiles: 184 VGPRs with
-// the run-time count, 168 compiled). Other counts run as the next larger one or, grouped, in the run-time form.
+// chunk's LDS reads and MFMAs are one straight block (4 slices of 40 to 2,000 orientations x 18 angles x 131 rows, 5 tiles,
+// adjoint with the run-time count / compiled: fp16 129 / 101 us, residual 85 / 85). Other counts run as the next larger
+// one or, grouped, in the run-time form.
 #define DFM_MT(MT, CALL)                                                                                           \
   switch (MT) {                                                                                                    \
     case 2: { constexpr int N = 2; CALL; break; }                                                                  \

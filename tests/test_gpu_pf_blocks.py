@@ -101,3 +101,36 @@ def test_block_products_at_tile_edges(my, K, CP, ksplit, precision):
         ref, mag = _product(datas, pfs.transpose(0, 2, 1), precision)
         assert np.all(np.abs(back[:, :, :K] - 2.0 * ref) <= rel * 2.0 * mag)
         assert np.all(back[:, :, K:] == 0.0)
+
+
+@pytest.mark.parametrize("precision", list(MODES))
+@pytest.mark.parametrize("my,K,CP", [(1, 1, 1), (17, 12, 33), (40, 33, 31), (103, 95, 70), (131, 20, 5)])
+def test_values_beside_the_columns_stay_out(my, K, CP, precision):
+    """NaN in the sinogram's columns beyond the orientations, in the data rows of other angles and behind the last row:
+    the chunk with fewer than 32 columns takes in none of them."""
+    import torch
+    print(f"case pf blocks padding my={my} K={K} CP={CP} {precision}", flush=True)
+    R, P = 4, 1
+    rng = np.random.default_rng(my + K)
+    pf = np.where(rng.random((R, K, CP)) < 0.4, rng.random((R, K, CP)), 0.0).astype(np.float32)
+    ptr, pos, val, inv, st = _store(torch.from_numpy(pf).cuda(), precision, P)
+    om = torch.tensor([1, 3], dtype=torch.int32, device="cuda")
+    sks = (K + 3) // 4 * 4 + 8
+    sino = np.full((3, my, sks), np.nan, np.float32)         # one matrix more than the angle list has
+    sino[:2, :, :K] = rng.random((2, my, K)) - 0.3
+    data = np.full((R + 1, my, CP), np.nan, np.float32)
+    data[[1, 3]] = rng.random((2, my, CP)) - 0.3
+    d_sino, d_data = torch.from_numpy(sino).cuda(), torch.from_numpy(data).cuda()
+    rel = 3 * (max(K, CP) + 4) * 2.0 ** -23                  # as above
+    for waves in (0, 32):
+        out = torch.full((R, my, CP), 7.0, device="cuda")
+        _lib.call("dfm_pfblk_forward", _lib.ptr(d_sino), sks, K, _lib.ptr(ptr), _lib.ptr(pos), _lib.ptr(val),
+                  MODES[precision] + waves, _lib.ptr(inv), P, _lib.ptr(om), 2, my, CP, _lib.ptr(out), None, 1, 0, st)
+        ref, mag = _product(sino[:2, :, :K], pf[[1, 3]], precision)
+        assert np.all(np.abs(out.cpu().numpy()[[1, 3]] - ref) <= rel * mag)
+        back = torch.full((2, my, sks), np.nan, device="cuda")
+        _lib.call("dfm_pfblk_adjoint", _lib.ptr(d_data), _lib.ptr(ptr), _lib.ptr(pos), _lib.ptr(val),
+                  MODES[precision] + waves, _lib.ptr(inv), P, _lib.ptr(om), 2, my, CP, K, _lib.ptr(back), sks, 1.0, st)
+        back = back.cpu().numpy().astype(np.float64)
+        ref, mag = _product(data[[1, 3]], pf[[1, 3]].transpose(0, 2, 1), precision)
+        assert np.all(np.abs(back[:, :, :K] - ref) <= rel * mag) and np.all(back[:, :, K:] == 0.0)
