@@ -1,5 +1,6 @@
-"""The rule that picks the forward projection's kernel by size, on the CPU: the line sweep walks lines of both directions, so
-narrow images, whose longer side costs the walk and whose few pixels cost the table little, keep the table."""
+"""Rules by size, on the CPU. The forward projection's kernel: the line sweep walks lines of both directions, so narrow
+images, whose longer side costs the walk and whose few pixels cost the table little, keep the table. The block products'
+split: launches of few waves are split finer, for the walk is all there is."""
 import pytest
 
 from diffractom_amd.operator import SinglePhaseForwardOperator
@@ -18,3 +19,13 @@ def test_kernel_by_size(nx, ny, n_angles, kn, kernel):
     assert op._fwd_kernel({"pairs_ok": True}, n_angles, kn) == kernel
     assert op._fwd_kernel({"pairs_ok": False}, n_angles, kn) == "table"
     assert op._fwd_kernel(None, n_angles, kn) == "table"
+
+
+@pytest.mark.parametrize("my,n_ang,n_jb,n_kb,ks", [
+    (32, 3, 4, 17, 8), (103, 1, 12, 17, 8), (103, 10, 4, 17, 8), (32, 18, 4, 10, 5), (103, 10, 29, 7, 1), (103, 1, 4, 7, 3),
+    (103, 18, 29, 17, 1), (103, 18, 29, 47, 3), (103, 18, 29, 94, 7), (103, 18, 29, 929, 16), (131, 9, 29, 17, 1),
+    (131, 9, 8, 17, 7), (17, 1, 1, 1, 1), (17, 1, 1, 3, 1), (17, 1, 1, 4, 2), (17, 1, 1, 5000, 64)])
+def test_block_product_split(my, n_ang, n_jb, n_kb, ks):
+    op = object.__new__(SinglePhaseForwardOperator)
+    op.My, op.blk_variant = my, {}
+    assert op._blk_split(n_ang, {"n_jb": n_jb, "n_kb": n_kb}) == ks
