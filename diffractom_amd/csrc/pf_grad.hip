@@ -18,11 +18,11 @@
 // LDS (float64 atomics) and written per (angle, orientation); the per-workgroup sums of the global parameters go to
 // a partial array. dfm_pf_grad_reduce sums both over angles / workgroups in a fixed order.
 //
-// What bounds it: load latency (waves wait 79 % of their cycles, VALU 27 -> 39 % busy). So an axis is loaded while the
+// What bounds it: load latency (waves wait 80 % of their cycles, VALU 36 % of the time). So an axis is loaded while the
 // one before is evaluated, the directions' derivatives are read once per node and multiply the axes' summed n dg/dd
 // (instead of 12 loads per contributing axis), the dot's and the staging's loads go ahead, the global parameters' sums
-// stay in registers until the end (they were 64-way conflicts on one LDS word), and 128 VGPRs keep four workgroups on a
-// CU (142 without the limit: 3; 1.46 -> 0.96 ms with the sums). 60 angles x 1,000 orientations x 67 rows, five rings:
+// stay in registers until the end (they were 64-way conflicts on one LDS word), and 128 VGPRs (27 spilled) keep four
+// workgroups on a CU (142 without the limit: 3; 1.46 -> 0.96 ms with the sums). 60 angles x 1,000 orientations x 67 rows, five rings:
 // 1.76 -> 0.96 ms.
 #include "pf_cand.h"
 

@@ -16,7 +16,8 @@
 // detector positions; with an entry per wave-instruction (two v_readlane, an add and 4-byte reads each) they cost 4
 // times (3 + NB), and that issue rate bounded the kernel: 9899 orientations x 180 angles x 900 segments x 103 rows, 6.2 %
 // fill (9.9e7 entries), forward with its split in two and transposes 2.47 -> 1.77 ms, adjoint 2.05 -> 1.30. VALU issue
-// still bounds it: a third of it entries, the rest the visits, their rounding to 4 entries and the staging. Rows whose
+// (62 % of the time at 2.4 GHz: a third of it entries, the rest the visits, their rounding to 4 entries and the staging) and
+// the waits of the visits' chains (54 % of the waves' cycles) bound it now. Rows whose
 // entries run out in a chunk before the others' of their quad read a zero operand. The first two windows of a visit are
 // loaded one visit ahead.
 //

@@ -1246,10 +1246,10 @@ class SinglePhaseForwardOperator:
         """Pick each product's fastest kernel variant by timing it on this operator's shapes (HIP events, median of
         reps after 2 warm-up launches), as the reference times its tiled and plain projectors
         (parallel_radon.py:240-281). Every candidate computes the same values (up to float32 summation order).
-        Candidates: forward projection (line sweeps with one or two rays per thread, pixel bands, geometry table
-        with 4 or 8 entries fetched ahead, staged in LDS or not, capped occupancy), backprojection with the SPDHG
-        update (4x4 and 8x8 tiles, 4, 8 or 16 angles staged per pass, 1-8 channel blocks per workgroup), the PF
-        products (block workgroup size and k split, CSR forms).
+        Candidates: forward projection (the line sweep with its lines loaded into LDS, in both layouts, its ranges by
+        size; register-staged sweeps with one or two rays per thread, pixel bands, geometry table staged in LDS),
+        backprojection with the SPDHG update (matrix cores; 8x8 tiles with 8 angles per pass and 1-4 channel blocks per
+        workgroup, two 4x4 forms), the PF products (block workgroup size and k split, CSR forms).
         Returns {product: (choice, {candidate: ms})} and keeps it in self.tuning."""
         if self.omega_subsets is None:
             self.set_omega_subsets(10)
