@@ -1071,11 +1071,11 @@ class SinglePhaseForwardOperator:
 
     def _lines_variant(self, tab, kn):
         """(line ranges, duplicated layout) of the line sweep: radon_variant["fwd_lines"] (ranges + 128 for the
-        duplicated layout, 0 ranges: by size) if set by hand or by autotune, which sets the layout alone (the ranges
-        that suit one subset are too many for all angles), else by size. The duplicated layout while two workgroups of
-        it fit a CU's LDS (128 pixels: 99 x 99 x 29760 x 18 angles 0.82 against 0.89 ms; 256 pixels, one workgroup: 1.62
-        against 1.20). With fewer workgroups than CUs the lines are split for two workgroups per CU, in ranges of 8
-        lines or more along the longer side and at most 12 (99 x 99 x 18 angles: 576 orientations 109 -> 46 us, 2048 117 -> 92 us; 5056, 316
+        duplicated layout, 0 ranges: by size) if set by hand, else by size, also by autotune (the ranges that suit one
+        subset are too many for all angles). The duplicated layout while two workgroups of it fit a CU's LDS (128
+        pixels: 99 x 99 x 29760 x 18 angles 0.82 against 0.89 ms; 256 pixels, one workgroup: 1.62 against 1.20). With
+        fewer workgroups than CUs the lines are split for two workgroups per CU, in ranges of 8 lines or more along the
+        longer side and at most 12 (99 x 99 x 18 angles: 576 orientations 109 -> 46 us, 2048 117 -> 92 us; 5056, 316
         workgroups, 178 -> 198)."""
         n = max(self.Nx, self.Ny)
         v = self.radon_variant.get("fwd_lines")
@@ -1174,8 +1174,10 @@ class SinglePhaseForwardOperator:
             cands = {}
             sl = _lib.load().dfm_radon_sweep_lines(self.Nx, self.Ny)
             if tab["pairs_ok"] and max(self.Nx, self.Ny) <= 256:
-                # the line sweep first: the fastest at every measured configuration but small images
-                cands.update({"lines" + "+dup" * d: ("lines", 128 * d) for d in (1, 0)})
+                # the line sweep first: the fastest at every measured configuration but small images. Its layout and
+                # ranges by size: on the dense random image timed here the layouts are 4 % apart either way, on a
+                # solver's image the duplicated one takes 0.64 ms and the other 0.75 (99 x 99 x 29760 x 18 angles)
+                cands["lines"] = ("lines", None)
             if sl and self.My <= 1024:         # 1024 rays per workgroup (512 for the 64-orientation form)
                 cands.update({f"sweep:{n}": ("sweep", n) for n in (4,) if n <= sl})
                 ln = max(self.Nx, self.Ny)
@@ -1246,8 +1248,8 @@ class SinglePhaseForwardOperator:
         """Pick each product's fastest kernel variant by timing it on this operator's shapes (HIP events, median of
         reps after 2 warm-up launches), as the reference times its tiled and plain projectors
         (parallel_radon.py:240-281). Every candidate computes the same values (up to float32 summation order).
-        Candidates: forward projection (the line sweep with its lines loaded into LDS, in both layouts, its ranges by
-        size; register-staged sweeps with one or two rays per thread, pixel bands, geometry table staged in LDS),
+        Candidates: forward projection (the line sweep with its lines loaded into LDS, its layout and ranges by size;
+        register-staged sweeps with one or two rays per thread, pixel bands, geometry table staged in LDS),
         backprojection with the SPDHG update (matrix cores; 8x8 tiles with 8 angles per pass and 1-4 channel blocks per
         workgroup, two 4x4 forms), the PF products (block workgroup size and k split, CSR forms).
         Returns {product: (choice, {candidate: ms})} and keeps it in self.tuning."""
