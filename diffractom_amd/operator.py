@@ -679,16 +679,16 @@ class SinglePhaseForwardOperator:
         pipeline fill, and its partial sums cost more to write and add up than the added waves give. 18 angles of 103
         rows and 8 segment blocks, 16 partial sums / this rule: 47 chunks 72.5 / 48.2 us (3 sums), 17 chunks 46.8 /
         33.6 (1 sum), 94 chunks 83 / 68 (7 sums); 310 and 929 chunks keep 16 (157, 377). Few waves leave most of the chip
-        idle, and the walk is all there is: up to 1024 waves (128 with less than 8 chunks) in up to 8 sums of 2 chunks or
-        more (us for 1 / 4 / 8 sums, fp16 x 103 rows: 17 chunks 12 waves 37 / 25 / 23, 40 waves residual 26 / 16 / 15;
-        10 chunks 72 waves x 32 rows 11.4 / 10.1 / 9.6; 7 chunks 290 waves 16.5 / 22 / 27). Over 240 shapes of 7 to 47
-        chunks it is 3 % from the best split of each (with 12 chunks for all: 29 %). The FP32 chains are longer than
+        idle, and the walk is all there is: from 8 chunks on, up to 1024 waves in up to 8 sums of 2 chunks or more (us for
+        1 / 4 / 8 sums, fp16 x 103 rows: 17 chunks 12 waves 37 / 25 / 23, 40 waves residual 26 / 16 / 15; 10 chunks 72
+        waves x 32 rows 11.4 / 10.1 / 9.6; 7 chunks 4 waves 10.8 / 9.9 / 10.0, 290 waves 16.5 / 22 / 27). Over 240 shapes
+        of 7 to 47 chunks it is 4 % from the best split of each (with 12 chunks for all: 29 %). The FP32 chains are longer than
         with 16 sums, which the operands' rounding hides: against the products in 64 bits, 543 orientations in 16 sums /
         in one, residual 1.686e-6 / 1.689e-6, fp16 1.143e-4 and bf16 9.24e-4 in both."""
         tiles = -(-self.My // 16)
         n_yg = -(-tiles // 8)
         waves, n = n_ang * n_yg * blk["n_jb"], blk["n_kb"]
-        few = min(n // 2, (1024 if n >= 8 else 128) // waves, 8)
+        few = min(n // 2, 1024 // waves, 8) if n >= 8 else 1
         return int(max(1, min(64, max(n // 12, few), -(-int(self.blk_variant.get("fwd_waves", 8192)) // waves))))
 
     def _blk_forward(self, ib, sino, data, subset, accumulate):
