@@ -685,6 +685,8 @@ int dfm_pfblk_adjoint(const float* data, const int32_t* ptr, const uint16_t* pos
                 "dfm_pfblk_adjoint: mode %d (0 bf16, 1 bf16 residual, 2 fp16 with ring scales)", mode);
   DFM_CHECK_ARG(n_ang > 0 && my > 0 && cp > 0 && kb > 0 && sks >= kb && (sks & 3) == 0,
                 "dfm_pfblk_adjoint: bad sizes (n_ang %d, My %d, CP %d, Kb %d, stride %d)", n_ang, my, cp, kb, sks);
+  DFM_CHECK_ARG((int64_t)(my < 32 ? my : 32) * cp < (int64_t)1 << 30,
+                "dfm_pfblk_adjoint: data rows of %d floats (32 of them pass 4 GiB)", cp);
   BlkArgs p{};
   p.blk_local = local;
   p.n_kb = (kb + 31) / 32;

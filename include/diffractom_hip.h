@@ -287,7 +287,7 @@ int dfm_mfma_grouped(int32_t forward, const dfm_mfma_desc* descs, const int32_t*
  * + lo*hi), 2 fp16 (val fp16; ring_inv[p] = 1 / ring_scale[p]; the y-side operand scaled by a power of two per row
  * and chunk of 32); + 16: the blocks are indexed by the position a in the angle list (a generated PF of just these
  * angles, dfm_pfgen) instead of by omegas[a]; + 32: 8 waves per workgroup; + 128: accepted, changes nothing. FP32
- * accumulation. */
+ * accumulation. 32 rows of the source (sks or cp floats each) must stay below 4 GiB. */
 int dfm_pfblk_count(const float* pf, int32_t* counts, int32_t R, int32_t km, int32_t kb, int32_t cp,
                     dfm_stream_t stream);
 int dfm_pfblk_fill(const float* pf, const int32_t* ptr, uint16_t* pos, void* val, int32_t fp16,

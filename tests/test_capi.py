@@ -47,3 +47,18 @@ def test_argument_errors_are_status_codes(lib):
     with pytest.raises(ValueError, match="ntap"):
         _lib.call("dfm_radon_backward", ctypes.c_void_p(8), ctypes.c_void_p(8), ctypes.c_void_p(8), 4, 4, 5, 3, 8,
                   0, 8, 8, 7, None)
+
+
+@pytest.mark.parametrize("my,row,refused", [(32, 1 << 25, True), (100, 1 << 26, True), (31, 1 << 26, True), (32, 1 << 24, False),
+                                            (1, 1 << 26, False)])
+def test_block_products_refuse_rows_beyond_their_buffers(lib, my, row, refused):
+    """32 source rows of 4 GiB or more do not fit a buffer's 32-bit offsets: an argument error in both directions (no angle
+    in the list otherwise: an error as well, and nothing is launched)."""
+    from diffractom_amd import _lib
+    p = ctypes.c_void_p(64)
+    n_ang = 1 if refused else 0
+    for match, args in (("sinogram rows", ("dfm_pfblk_forward", p, row, row, p, p, p, 1, None, 0, p, n_ang, my, 32, p, p, 1, 0,
+                                           None)),
+                        ("data rows", ("dfm_pfblk_adjoint", p, p, p, p, 1, None, 0, p, n_ang, my, row, 32, p, 32, 1.0, None))):
+        with pytest.raises(ValueError, match=match if refused else "bad sizes"):
+            _lib.call(*args)
